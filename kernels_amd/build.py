@@ -41,7 +41,7 @@ HIP_FLAGS = [
 ]
 
 LIB_SOURCES = ["prk_api.hip", "sweep_f64.hip", "sweep_f32.hip", "sweep_bf16.hip",
-               "batch.hip", "server.hip", "autotune.hip", "transpose.hip"]
+               "pass_f64.hip", "pass_f32.hip", "pass_bf16.hip", "batch.hip", "server.hip", "autotune.hip", "transpose.hip"]
 # command-line drivers: executable -> source
 CLIS = {"prk-stencil": "prk_cli.cpp", "prk-transpose": "prk_transpose_cli.cpp"}
 

@@ -14,6 +14,7 @@
 #include <string>
 #include <vector>
 
+#include "pass.hpp"
 #include "prk_internal.hpp"
 #include "sweep.hpp"
 
@@ -98,6 +99,34 @@ int launch_sweep(const SweepPlan &p, const void *in, void *in_next, void *out, h
     case F64: return launch_sweep_f64(p, in, in_next, out, s);
     case F32: return launch_sweep_f32(p, in, in_next, out, s);
     case BF16: return launch_sweep_bf16(p, in, in_next, out, s);
+    }
+    return set_error(PRK_EINVAL, "unknown dtype %d", p.dtype);
+}
+
+template <int DT>
+static bool pass_built_dtype(int pattern, int radius)
+{
+    constexpr bool ok[2][8] = {
+        {pass_ok<DT, STAR, 1>(), pass_ok<DT, STAR, 2>(), pass_ok<DT, STAR, 3>(), pass_ok<DT, STAR, 4>(),
+         pass_ok<DT, STAR, 5>(), pass_ok<DT, STAR, 6>(), pass_ok<DT, STAR, 7>(), pass_ok<DT, STAR, 8>()},
+        {pass_ok<DT, GRID, 1>(), pass_ok<DT, GRID, 2>(), pass_ok<DT, GRID, 3>(), pass_ok<DT, GRID, 4>(),
+         pass_ok<DT, GRID, 5>(), pass_ok<DT, GRID, 6>(), pass_ok<DT, GRID, 7>(), pass_ok<DT, GRID, 8>()}};
+    return ok[pattern == GRID][radius - 1];
+}
+
+bool pass_built(int pattern, int radius, int dtype)
+{
+    return dtype == F64 ? pass_built_dtype<F64>(pattern, radius)
+           : dtype == F32 ? pass_built_dtype<F32>(pattern, radius)
+                          : pass_built_dtype<BF16>(pattern, radius);
+}
+
+int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
+{
+    switch (p.dtype) {
+    case F64: return launch_pass_f64(p, sweeps, in, in_next, out, s);
+    case F32: return launch_pass_f32(p, sweeps, in, in_next, out, s);
+    case BF16: return launch_pass_bf16(p, sweeps, in, in_next, out, s);
     }
     return set_error(PRK_EINVAL, "unknown dtype %d", p.dtype);
 }
@@ -662,11 +691,27 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
         (void)hipEventDestroy(e0);
         return rc;
     }
+    // Sweep 0 runs by itself; the timed sweeps run in `passes` passes over the
+    // grid (pass.hpp) of nearly equal length.  The final in must end in the
+    // buffer that one sweep per pass would leave it in, so the number of
+    // passes is odd or even as the number of sweeps is.  A tiling override
+    // asks for the sweep kernel itself: one sweep per pass then.
+    const bool overridden = g_rows_per_wave > 0 || g_variant_override >= 0 || g_order >= 0 || g_wgs_per_cu >= 0;
+    int passes = iterations;
+    if (!overridden && pass_built(pattern, radius, dtype)) {
+        passes = (iterations + kMaxPassSweeps - 1) / kMaxPassSweeps;
+        passes += (passes ^ iterations) & 1;
+    }
     void *bufs[2] = {buf0, buf1};
     int cur = 0;
-    for (int it = 0; it <= iterations && rc == PRK_OK; ++it) {
+    for (int it = 0, done = 0; it <= passes && rc == PRK_OK; ++it) {
         if (it == 1) rc = check_hip(hipEventRecord(e0, s), "event record");
-        if (rc == PRK_OK) rc = launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s);
+        // sweeps left, spread over the passes left
+        const int sweeps = it == 0 ? 1 : (iterations - done) / (passes - it + 1);
+        if (rc == PRK_OK)
+            rc = sweeps == 1 ? launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s)
+                             : launch_pass(p, sweeps, bufs[cur], bufs[cur ^ 1], out, s);
+        if (it > 0) done += sweeps;
         cur ^= 1;
     }
     if (rc == PRK_OK) rc = check_hip(hipEventRecord(e1, s), "event record");
