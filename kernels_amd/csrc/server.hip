@@ -130,6 +130,7 @@ struct prk_server {
     size_t h_tab_cap[2] = {0, 0};
     size_t norm_off[2] = {0, 0};  // finishing requests' norms in the slot's tables
     hipGraphExec_t exec[2] = {nullptr, nullptr};
+    std::vector<std::pair<int, int>> exec_launches[2];  // class and workgroups of each launch in exec
     // FP64 shadow solves: error kernels on their own stream, partials and the
     // result on the device, the result in pinned memory, a count per class
     hipStream_t aux = nullptr;
@@ -436,8 +437,19 @@ int build_window(prk_server *s, long long w)
     const int rc2 = check_hip(hipStreamEndCapture(s->capture, &g), "server end capture");
     if (!rc) rc = rc2;
     // The slot's exec last ran window w-2, which has finished.  Where the new
-    // graph has its topology (the same classes, the same rounds each) the
-    // exec takes the new kernel arguments in place; otherwise it is replaced.
+    // graph has its launches (the same kernels, in the same order, with the
+    // same workgroups) the exec takes the new kernel arguments in place;
+    // otherwise it is replaced.  A graph of the same topology is not enough:
+    // an exec updated to another number of workgroups does not launch that
+    // number.
+    std::vector<std::pair<int, int>> sig;
+    for (const auto &v : launches)
+        for (const Launch &l : v) sig.push_back({l.cls, l.blocks});
+    if (s->exec[slot] && s->exec_launches[slot] != sig) {
+        (void)hipGraphExecDestroy(s->exec[slot]);
+        s->exec[slot] = nullptr;
+    }
+    s->exec_launches[slot] = sig;
     bool updated = false;
     if (!rc && s->exec[slot]) {
         hipGraphNode_t bad = nullptr;

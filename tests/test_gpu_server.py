@@ -161,3 +161,19 @@ def test_shadow_solves_report_error_vs_f64(gpu, oracle):
         assert abs(got["normwise"] - nw) <= 1e-12 * nw, (s, got, nw)
         assert r["t_admit"] <= r["t_done"]
     srv.close()
+
+
+def test_windows_of_equal_topology_keep_their_own_launches(gpu, oracle):
+    # One request at a time, every one with the same number of stages but
+    # another stencil or size: each window's graph has the topology of the
+    # one that ran in its slot before and other kernels, or other numbers of
+    # workgroups, in its nodes.  Every result is still the oracle's.
+    srv = Server(budget_bytes=1 << 30)
+    for i in range(16):
+        s = (i % 2 if i < 8 else 0, 1 + (i // 2) % 3 if i < 8 else 2, F64, 90 + 40 * (i * 5 % 7), 4, 1, 500 + i)
+        print(f"request {i}: {s}", flush=True)
+        ids, res = run_all(srv, [s])
+        out, _, norm = ref_solve(oracle, s)
+        assert np.array_equal(srv.fetch(ids[0]).view(np.uint8), out.view(np.uint8)), s
+        assert abs(res[ids[0]]["norm"] - norm) <= 1e-13 * abs(norm), s
+    srv.close()
