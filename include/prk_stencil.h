@@ -226,14 +226,15 @@ int prk_tuning_load(const char *path);
  * grid: initial values, iterations+1 fused sweeps, L1 norm.  A batch holds
  * many solves of any sizes, patterns, radii (1..8), iteration counts and
  * storage types; prk_batch_create allocates all their grids in one device
- * pool (rows padded to 128 bytes; padding columns are scratch), cuts a
- * sliding-window schedule into rounds (one stage of each active solve per
- * round, one launch per round and (storage type, pattern, radius) class
- * over the tiles of its solves) and captures the whole run in a hipGraph,
- * one branch per class.  Every solve's arithmetic is that of the
- * single-grid sweep, so each result is the same whatever else is in the
- * batch.  rows_per_tile: tile height (0 = the height prk_batch_autotune
- * chose for the solve's key, else 32).  flags: 0, or PRK_BATCH_PERSISTENT for the
+ * pool (rows padded to 128 bytes; padding columns are scratch) and captures
+ * the whole run in a hipGraph with a branch per (storage type, pattern,
+ * radius) class: a launch that runs up to 64 sweeps of all its solves where
+ * the stencil's window fits the registers; else a sliding-window schedule
+ * cut into rounds (one stage of each active solve per round, one launch per
+ * round).  Every solve's arithmetic is that of the single-grid sweep, so
+ * each result is the same whatever else is in the batch.  rows_per_tile:
+ * tile height of the sweep-by-sweep stages (0 = the height
+ * prk_batch_autotune chose for the solve's key, else 32).  flags: 0, or PRK_BATCH_PERSISTENT for the
  * single-launch tile-queue form, which is disabled (it hung on MI355X) and
  * returns PRK_EINVAL.
  *   prk_batch_run     enqueue one run of every solve on `stream`

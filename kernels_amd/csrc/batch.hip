@@ -1,9 +1,12 @@
 // Host side of the batched solve path: one device pool for every solve's
-// grids, a sliding-window schedule cut into rounds (a round holds at most one
-// stage of each solve), one launch per round, all rounds of a storage type on
-// one stream and the storage types on parallel branches of one captured
-// hipGraph.  Also the one-grid-per-launch baseline that runs the same solves
-// through the single-grid sweep.
+// grids and one captured hipGraph for the run.  Solves whose stencil has a
+// pass kernel are initialised by one launch over all of them; then each
+// class (storage type, pattern, radius) has a branch with a launch per pass.
+// Classes without one go through a sliding-window schedule cut into rounds
+// (a round holds at most one stage of each solve), one launch per round.
+// The branches join in one launch that reduces every solve's norm partials.
+// Also the one-grid-per-launch baseline that runs the same solves through
+// the single-grid sweep.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -25,7 +28,7 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 int vec_of(int dt) { return dt == F64 ? 2 : dt == F32 ? 4 : 8; }
 
-// Rows per tile: each tile re-reads 2R halo rows and pays a pipeline
+// Rows per tile of the row-by-row stages: each tile re-reads 2R halo rows and pays a pipeline
 // prologue, so batched tiles are taller than the single-grid row blocks
 // (32 measured best for the 4096-grid mix on MI355X).
 int default_tile_rows(int) { return 32; }
@@ -83,6 +86,7 @@ struct prk_batch {
     // classes: storage type x pattern x radius (1..8)
     static constexpr int kClasses = 3 * 2 * kBatchMaxRadius;
     std::vector<Round> rounds[kClasses];
+    Round init{0, 0, 0};  // the solves that have passes
     long long total_tiles = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -109,12 +113,41 @@ int validate_solve(const prk_solve &s)
     return PRK_OK;
 }
 
-int stage_tiles(const BGrid &g, int stage) { return stage == g.iters + 3 ? 1 : g.ntiles; }
+// Workgroup entries of one stage of solve g.
+void push_work(std::vector<RWork> &work, Round &r, const BGrid &bg, int g, int stage)
+{
+    const int tiles = batch_stage_tiles(bg, stage);
+    for (int t0 = 0; t0 < tiles; t0 += kWavesPerBlock) work.push_back(RWork{g, stage, t0});
+    r.blocks += (tiles + kWavesPerBlock - 1) / kWavesPerBlock;
+    r.tiles += tiles;
+}
+
+// Passes: pass p of every solve that has one in one launch, the solves with
+// the most sweeps first (a wave's time goes with its solve's sweeps, and the
+// launch ends with its last wave).
+void schedule_passes(const std::vector<int> &ids, const std::vector<BGrid> &grids, std::vector<RWork> &work,
+                     std::vector<Round> &rounds)
+{
+    std::vector<int> order(ids);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return grids[a].iters > grids[b].iters; });
+    std::vector<int> stage(grids.size(), 1);
+    for (bool any = true; any;) {
+        any = false;
+        Round r{work.size(), 0, 0};
+        for (int g : order) {
+            if (stage[g] > grids[g].iters + 1) continue;
+            push_work(work, r, grids[g], g, stage[g]);
+            stage[g] = batch_next_stage(grids[g], stage[g]);
+            any = true;
+        }
+        if (any) rounds.push_back(r);
+    }
+}
 
 // Sliding window: keep enough solves active that a round of their next
 // stages holds about `target` tiles; each round takes one stage of every
-// active solve; a solve leaves after its final-norm stage and the next one
-// in submission order takes its place.
+// active solve; a solve leaves after its norm-partials stage and the next
+// one in submission order takes its place.
 void schedule_rounds(const std::vector<int> &ids, const std::vector<BGrid> &grids, long long target,
                      std::vector<RWork> &work, std::vector<Round> &rounds)
 {
@@ -131,11 +164,9 @@ void schedule_rounds(const std::vector<int> &ids, const std::vector<BGrid> &grid
         Round r{work.size(), 0, 0};
         std::vector<int> keep;
         for (int g : active) {
-            const int tiles = stage_tiles(grids[g], stage[g]);
-            for (int t0 = 0; t0 < tiles; t0 += kWavesPerBlock) work.push_back(RWork{g, stage[g], t0});
-            r.blocks += (tiles + kWavesPerBlock - 1) / kWavesPerBlock;
-            r.tiles += tiles;
-            if (++stage[g] <= grids[g].iters + 3) keep.push_back(g);
+            push_work(work, r, grids[g], g, stage[g]);
+            stage[g] = batch_next_stage(grids[g], stage[g]);
+            if (stage[g] < batch_last_stage(grids[g])) keep.push_back(g);
             else in_flight -= grids[g].ntiles;
         }
         rounds.push_back(r);
@@ -182,6 +213,43 @@ int launch_round_pr(int radius, const RoundArgs &a, unsigned blocks, hipStream_t
 namespace prk {
 
 int batch_class_of(const prk_solve &s) { return (s.dtype * 2 + s.pattern) * kBatchMaxRadius + (s.radius - 1); }
+
+// Initial values of every solve that has passes, over its pass tiles.
+__global__ __launch_bounds__(kThreads) void batch_init_kernel(RoundArgs a)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const RWork wk = a.work[blockIdx.x];
+    const BGrid &g = a.grids[wk.grid];
+    const int tile = wk.tile0 + wave;
+    if (tile >= g.pass_tiles) return;
+    int strip, r0;
+    pass_tile_at(g, tile, strip, r0);
+    const int r1 = min(r0 + g.pass_rows, g.n);
+    if (g.dtype == F64) init_tile<F64, false>(g, strip * SweepGeom<F64, 1>::SW, r0, r1, lane);
+    else if (g.dtype == F32) init_tile<F32, false>(g, strip * SweepGeom<F32, 1>::SW, r0, r1, lane);
+    else init_tile<BF16, false>(g, strip * SweepGeom<BF16, 1>::SW, r0, r1, lane);
+}
+
+// The final norms, one workgroup per solve: each wave sums every fourth run
+// of 64 partials, the waves' sums are added in order.
+__global__ __launch_bounds__(kThreads) void batch_norm_kernel(const BGrid *grids)
+{
+    const BGrid &g = grids[blockIdx.x];
+    const int partials = g.npartials;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    DDv acc{0.0, 0.0};
+    for (int k = threadIdx.x; k < partials; k += kThreads) acc = dd_add_dev(acc, g.partials[k]);
+    acc = wave_reduce_dd(acc);
+    __shared__ DDv waves[kWavesPerBlock];
+    if (lane == 0) waves[wave] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        acc = waves[0];
+        for (int w = 1; w < kWavesPerBlock; ++w) acc = dd_add_dev(acc, waves[w]);
+        const long long wd = g.n - 2 * g.radius;
+        *g.norm = (acc.hi + acc.lo) / (double)(wd * wd);
+    }
+}
 
 // Fixed-order block reduction of four values (max, then three sums).
 __device__ inline void err_block_reduce(double (&v)[4], double *out)
@@ -297,7 +365,6 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
         g.n = s.n;
         g.pattern = s.pattern;
         g.radius = s.radius;
-        g.iters = s.iterations;
         g.rows = std::min(s.n, tile_rows_for(s, rows_per_tile));
         g.strips = (s.n + 64 * V - 1) / (64 * V);
         g.ntiles = g.strips * ((s.n + g.rows - 1) / g.rows);
@@ -305,7 +372,8 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
         g.seed = s.seed;
         offs[i] = off;
         off += 3 * align_up((size_t)s.n * (size_t)g.pitch * dtype_size(s.dtype), 256);
-        partial_total += (size_t)g.ntiles;
+        batch_set_passes(g, s, kBatchPassSweeps, kBatchPassRows);
+        partial_total += (size_t)g.npartials;
     }
     b->pool_bytes = off;
     rc = check_hip(hipMalloc(&b->pool, off), "batch grid pool");
@@ -333,8 +401,16 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
         cwork[c] += w;
         all_work += w;
     }
+    for (int i = 0; i < count; ++i)
+        if (batch_has_passes(b->grids[i])) push_work(work, b->init, b->grids[i], i, 1);
+    b->total_tiles = b->init.tiles;
     for (int c = 0; c < prk_batch::kClasses; ++c) {
         if (ids[c].empty()) continue;
+        if (batch_has_passes(b->grids[ids[c][0]])) {
+            schedule_passes(ids[c], b->grids, work, b->rounds[c]);
+            for (const Round &r : b->rounds[c]) b->total_tiles += r.tiles;
+            continue;
+        }
         const long long target = std::max<long long>(1024, g_round_tiles * cwork[c] / std::max<long long>(all_work, 1));
         schedule_rounds(ids[c], b->grids, target, work, b->rounds[c]);
         for (const Round &r : b->rounds[c]) b->total_tiles += r.tiles;
@@ -363,7 +439,7 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
     size_t pk = 0;
     for (int i = 0; i < count; ++i) {
         b->grids[i].partials = parts + pk;
-        pk += (size_t)b->grids[i].ntiles;
+        pk += (size_t)b->grids[i].npartials;
         b->grids[i].norm = b->d_norms + i;
     }
     rc = check_hip(hipMemcpy(b->d_grids, b->grids.data(), sizeof(BGrid) * count, hipMemcpyHostToDevice), "grids");
@@ -375,7 +451,12 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
         return rc;
     }
 
-    // capture: fork one branch per class present, its rounds in order, join
+    // capture: initialise, fork one branch per class present (the most work
+    // first), its launches in order, join, final norms
+    std::vector<int> classes;
+    for (int c = 0; c < prk_batch::kClasses; ++c)
+        if (!b->rounds[c].empty()) classes.push_back(c);
+    std::stable_sort(classes.begin(), classes.end(), [&](int x, int y) { return cwork[x] > cwork[y]; });
     rc = check_hip(hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking), "batch stream");
     if (!rc) rc = check_hip(hipEventCreateWithFlags(&b->done, hipEventDisableTiming), "batch event");
     if (!rc) rc = check_hip(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming), "batch event");
@@ -386,9 +467,14 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
     }
     if (!rc) rc = check_hip(hipStreamBeginCapture(b->capture, hipStreamCaptureModeThreadLocal), "begin capture");
     if (!rc) {
-        rc = check_hip(hipEventRecord(b->fork, b->capture), "fork");
-        for (int c = 0; c < prk_batch::kClasses && !rc; ++c) {
-            if (b->rounds[c].empty()) continue;
+        if (b->init.blocks) {
+            hipLaunchKernelGGL(batch_init_kernel, dim3((unsigned)b->init.blocks), dim3(kThreads), 0, b->capture,
+                               RoundArgs{b->d_grids, b->d_work + b->init.first_work});
+            rc = check_hip(hipGetLastError(), "batch init launch");
+        }
+        if (!rc) rc = check_hip(hipEventRecord(b->fork, b->capture), "fork");
+        for (int c : classes) {
+            if (rc) break;
             rc = check_hip(hipStreamWaitEvent(b->branch[c], b->fork, 0), "fork wait");
             for (const Round &r : b->rounds[c]) {
                 if (rc) break;
@@ -397,6 +483,11 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
             }
             if (!rc) rc = check_hip(hipEventRecord(b->join[c], b->branch[c]), "join");
             if (!rc) rc = check_hip(hipStreamWaitEvent(b->capture, b->join[c], 0), "join wait");
+        }
+        if (!rc) {
+            hipLaunchKernelGGL(batch_norm_kernel, dim3((unsigned)count), dim3(kThreads), 0, b->capture,
+                               (const BGrid *)b->d_grids);
+            rc = check_hip(hipGetLastError(), "batch norm launch");
         }
         hipGraph_t g = nullptr;
         const int rc2 = check_hip(hipStreamEndCapture(b->capture, &g), "end capture");
@@ -439,7 +530,7 @@ int prk_batch_output(const prk_batch *b, int idx, int which, void *host, size_t 
     const BGrid &g = b->grids[idx];
     const size_t es = dtype_size(b->solves[idx].dtype);
     if (bytes < (size_t)g.n * g.n * es) return set_error(PRK_EINVAL, "host buffer too small");
-    const void *src = which == 0 ? g.out : ((b->solves[idx].iterations + 1) % 2 ? g.buf1 : g.buf0);
+    const void *src = which == 0 ? g.out : (batch_final_buf(g) ? g.buf1 : g.buf0);
     return check_hip(hipMemcpy2D(host, (size_t)g.n * es, src, (size_t)g.pitch * es, (size_t)g.n * es, (size_t)g.n,
                                  hipMemcpyDeviceToHost),
                      "batch output copy");
@@ -451,7 +542,7 @@ int prk_batch_info(const prk_batch *b, long long *device_bytes, long long *tiles
     if (device_bytes) *device_bytes = (long long)b->pool_bytes;
     if (tiles) *tiles = b->total_tiles;
     if (launches) {
-        size_t l = 0;
+        size_t l = 1 + (b->init.blocks ? 1 : 0);  // final norms, init
         for (const auto &r : b->rounds) l += r.size();
         *launches = (int)l;
     }

@@ -1,25 +1,30 @@
 // Batched solves: many independent solves (grids of any size, star/grid,
 // radius 1..8, their own iteration counts) in a few launches.
 //
-// The host cuts the schedule into rounds; a round holds at most one stage of
-// each solve, so its tiles are independent and one plain launch runs them all
-// (a table gives each workgroup its solve, stage and tiles); stage order
-// within a solve comes from launch order.  Solves are grouped in classes of
-// one (storage type, pattern, radius), each with its own kernel and schedule
-// on its own branch of one captured hipGraph.  No wave ever waits on
-// another.  (A persistent form, one launch whose waves took tiles from
-// queues and waited on per-solve counters, hung on MI355X; it was removed and
-// the host refuses PRK_BATCH_PERSISTENT.)
+// A solve is a sequence of stages over its tiles: stage 0 initialises in,
+// stages 1..K+1 are its K+1 sweeps, stage K+2 computes the L1 norm partials
+// and stage K+3 reduces them.  Where the stencil has a pass kernel
+// (pass.hpp) one pass takes pass_sweeps sweeps: a solve then goes through
+// stages 1, 1 + pass_sweeps, 1 + 2 pass_sweeps, ..., the first pass starts
+// out from zeros and the last one leaves the norm partials, so stage K+2
+// falls away (batch_next_stage).  Pass p reads buffer p%2 and writes buffer
+// (p+1)%2.  A tile is one wavefront's share of a stage: 64*V columns of a
+// block of rows, processed by the same pass_tile() or wave_tile() as a
+// single grid, so a solve's arithmetic does not depend on what else is in
+// the launch.
 //
-// A solve is a sequence of stages over its tiles: stage 0 initialises in and
-// out, stages 1..K+1 are the K+1 fused sweeps (sweep k reads buffer k%2 and
-// writes buffer (k+1)%2), stage K+2 computes the L1 norm partials and stage
-// K+3 reduces them.  A tile is one wavefront's share of a stage: 64*V
-// columns of a block of rows, processed by the same wave_tile() as the
-// single-grid sweep, so a solve's arithmetic does not depend on what else is
-// in the launch.
+// Solves are grouped in classes of one (storage type, pattern, radius), each
+// with its own kernel.  One launch is one round: at most one stage of each
+// solve, so its tiles are independent (a table gives each workgroup its
+// solve, stage and tiles); stage order within a solve comes from launch
+// order.  No wave ever waits on another.  (A persistent form, one launch
+// whose waves took tiles from queues and waited on per-solve counters, hung
+// on MI355X; it was removed and the host refuses PRK_BATCH_PERSISTENT.)
 #pragma once
 
+#include <algorithm>
+
+#include "pass.hpp"
 #include "prk_stencil.h"
 #include "sweep.hpp"
 
@@ -44,19 +49,23 @@ struct DDv {
     double hi, lo;
 };
 
-// 32-byte aligned (96 bytes): every workgroup reads its grid's entry with
+// 32-byte aligned (128 bytes): every workgroup reads its grid's entry with
 // scalar loads at the start of a tile.
 struct alignas(32) BGrid {
     void *buf0, *buf1, *out;
     long long pitch;         // elements, 128-byte multiple (lib_pitch); padding may be written
-    int n, pattern, radius;
+    int n, pattern, radius, dtype;
     int iters;               // K: the solve runs K+1 sweeps
+    int pass_sweeps;         // sweeps of one pass (the last may have fewer)
     int rows;                // rows per tile
     int strips;              // ceil(n / 64V)
     int ntiles;              // strips * ceil(n / rows)
     int init_kind;
+    int pass_rows;           // rows per tile of a pass
+    int pass_tiles;          // strips * ceil(n / pass_rows)
+    int npartials;           // norm partials: pass_tiles, or ntiles without a pass kernel
     unsigned long long seed;
-    DDv *partials;           // ntiles norm partials
+    DDv *partials;           // the norm partials
     double *norm;            // result: L1 norm / (n-2R)^2
 };
 
@@ -86,8 +95,9 @@ __device__ inline DDv wave_reduce_dd(DDv v)
     return v;
 }
 
-// Stage 0: in = initial values, out = 0 over the tile (padding columns 0).
-template <int DT>
+// Stage 0: in = initial values over the tile (padding columns 0), and out = 0
+// if the first sweep does not set it (OUT).
+template <int DT, bool OUT>
 __device__ inline void init_tile(const BGrid &g, int c0, int r0, int r1, int lane)
 {
     typedef typename DTypeTraits<DT>::T T;
@@ -115,7 +125,7 @@ __device__ inline void init_tile(const BGrid &g, int c0, int r0, int r1, int lan
         }
         const unsigned off = (unsigned)(cm * ES);
         bstore16<0>(row_rsrc((T *)g.buf0 + (long long)r * g.pitch, row_bytes), off, x.v);
-        bstore16<0>(row_rsrc((T *)g.out + (long long)r * g.pitch, row_bytes), off, z.v);
+        if constexpr (OUT) bstore16<0>(row_rsrc((T *)g.out + (long long)r * g.pitch, row_bytes), off, z.v);
     }
 }
 
@@ -151,6 +161,47 @@ __device__ inline DDv norm_tile(const BGrid &g, int c0, int r0, int r1, int lane
     return wave_reduce_dd(DDv{sum, comp});
 }
 
+// Sweeps of one pass at most: in a batch, where a pass's traffic is already
+// small beside the arithmetic of this many; in the server, whose requests
+// take turns round by round and whose windows are a few rounds long.
+constexpr int kBatchPassSweeps = 64;
+constexpr int kServerPassSweeps = 6;
+
+// Rows of a batch's pass tiles: one group of rows per wave.  A pass loads
+// every group's window anew, so taller tiles save nothing but the partials,
+// and they leave small batches with few waves.  Measured on MI355X, 4, 8 and
+// 16 rows: 512 mixed solves of n up to 2048 6.71, 6.65, 6.74 ms; 300 of n up
+// to 300 0.34, 0.57, 0.89 ms; 64 of n up to 2048 1.56, 1.65, 1.85 ms.
+constexpr int kBatchPassRows = 4;
+
+__device__ inline void pass_tile_at(const BGrid &g, int tile, int &strip, int &r0)
+{
+    const int nrb = g.pass_tiles / g.strips;
+    strip = tile / nrb;
+    r0 = (tile - strip * nrb) * g.pass_rows;
+}
+
+// The pass that starts with sweep k, over pass tile `tile` (tiles run down
+// the strips: the waves of a workgroup share the rows their windows share).
+template <int DT, int P, int R>
+__device__ inline void pass_stage(const BGrid &g, int k, int tile, int lane)
+{
+    constexpr int V = DTypeTraits<DT>::V;
+    const int p = k / g.pass_sweeps, sweeps = min(g.pass_sweeps, g.iters + 1 - k);
+    int strip, r0;
+    pass_tile_at(g, tile, strip, r0);
+    const bool last = k + sweeps > g.iters;
+    NormSum ns;
+    pass_tile<DT, P, R, true>((p & 1) ? g.buf1 : g.buf0, (p & 1) ? g.buf0 : g.buf1, g.out, g.pitch, g.n,
+                              (strip * 64 + lane) * V, r0, min(r0 + g.pass_rows, g.n), sweeps, (int)g.pitch, k == 0,
+                              last, ns);
+    if (last) {
+        const DDv part = wave_reduce_dd(DDv{ns.sum, ns.comp});
+        if (lane == 0) g.partials[tile] = part;
+    }
+}
+
+// Sweep k as a stage of its own.
 template <int DT, int P, int R>
 __device__ inline void sweep_tile(const BGrid &g, int k, int c0, int r0, int r1, typename DTypeTraits<DT>::T *ring,
                                   int lane)
@@ -166,9 +217,7 @@ __device__ inline void sweep_tile(const BGrid &g, int k, int c0, int r0, int r1,
 // ---------------------------------------------------------------------------
 // Round form.  One launch = one round.  Every workgroup of the launch has a
 // work entry (solve, stage, first tile) and its four waves run four
-// consecutive tiles of that stage.  Stages: 0 init, 1..K+1 sweeps, K+2 norm
-// partials, K+3 the solve's final norm (one tile: reduces the partials in
-// tile order).
+// consecutive tiles of that stage.
 // ---------------------------------------------------------------------------
 struct RWork {
     int grid;
@@ -181,6 +230,16 @@ struct RoundArgs {
     const RWork *work;  // one entry per workgroup
 };
 
+// The final norm of a solve from its partials, by one wave.
+__device__ inline void final_norm(const BGrid &g, int lane)
+{
+    DDv acc{0.0, 0.0};
+    for (int k = lane; k < g.npartials; k += 64) acc = dd_add_dev(acc, g.partials[k]);
+    acc = wave_reduce_dd(acc);
+    const long long wd = g.n - 2 * g.radius;
+    if (lane == 0) *g.norm = (acc.hi + acc.lo) / (double)(wd * wd);
+}
+
 // One kernel per (storage type, pattern, radius): each keeps the registers
 // and LDS ring its own stencil needs.
 template <int DT, int P, int R>
@@ -189,37 +248,75 @@ __global__ __launch_bounds__(kThreads) void batch_round_kernel(RoundArgs a)
     typedef SweepGeom<DT, R> G;
     typedef typename G::T T;
     constexpr int SW = G::SW;
-    __shared__ __attribute__((aligned(16))) T lds[kWavesPerBlock][G::S * G::LR];
-    const int wave = threadIdx.x >> 6;
+    constexpr bool PASS = pass_ok<DT, P, R>();
+    constexpr int kRing = PASS ? 1 : G::S * G::LR;  // passes use no LDS
+    __shared__ __attribute__((aligned(16))) T lds[kWavesPerBlock][kRing];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const RWork wk = a.work[blockIdx.x];
     const BGrid &g = a.grids[wk.grid];
     const int norm_stage = g.iters + 2;
     const int tile = wk.tile0 + wave;
-    if (tile >= (wk.stage == norm_stage + 1 ? 1 : g.ntiles)) return;
+    if (wk.stage == norm_stage + 1) {
+        if (wave == 0) final_norm(g, lane);
+        return;
+    }
+    if constexpr (PASS) {
+        if (wk.stage > 0) {
+            if (tile < g.pass_tiles) pass_stage<DT, P, R>(g, wk.stage - 1, tile, lane);
+            return;
+        }
+    }
+    if (tile >= g.ntiles) return;
     const int rb = tile / g.strips;
     const int c0 = (tile - rb * g.strips) * SW;
     const int r0 = rb * g.rows;
     const int r1 = min(r0 + g.rows, g.n);
-    if (wk.stage == 0) {
-        init_tile<DT>(g, c0, r0, r1, lane);
+    if constexpr (PASS) {
+        init_tile<DT, false>(g, c0, r0, r1, lane);
+    } else if (wk.stage == 0) {
+        init_tile<DT, true>(g, c0, r0, r1, lane);
     } else if (wk.stage < norm_stage) {
         sweep_tile<DT, P, R>(g, wk.stage - 1, c0, r0, r1, lds[wave], lane);
-    } else if (wk.stage == norm_stage) {
+    } else {
         const DDv part = norm_tile<DT>(g, c0, r0, r1, lane);
         if (lane == 0) g.partials[tile] = part;
-    } else {
-        DDv acc{0.0, 0.0};
-        for (int k = lane; k < g.ntiles; k += 64) acc = dd_add_dev(acc, g.partials[k]);
-        acc = wave_reduce_dd(acc);
-        const long long wd = g.n - 2 * g.radius;
-        if (lane == 0) *g.norm = (acc.hi + acc.lo) / (double)(wd * wd);
     }
 }
 
 // Host helpers shared by the batch and the server (batch.hip).
 int batch_class_of(const prk_solve &s);  // (dtype, pattern, radius) class index
 constexpr int kBatchClasses = 3 * 2 * kBatchMaxRadius;
+// The solve's sweeps, how many of them a pass takes (passes of equal length,
+// the last perhaps shorter) and a pass's tiles.  Without a pass kernel each
+// sweep is a stage over the solve's ordinary tiles.
+inline void batch_set_passes(BGrid &g, const prk_solve &s, int max_sweeps, int rows)
+{
+    const int sweeps = s.iterations + 1;
+    const int passes = pass_built(s.pattern, s.radius, s.dtype) ? (sweeps + max_sweeps - 1) / max_sweeps : sweeps;
+    g.dtype = s.dtype;
+    g.iters = s.iterations;
+    g.pass_sweeps = (sweeps + passes - 1) / passes;
+    g.pass_rows = rows;
+    g.pass_tiles = g.strips * ((g.n + rows - 1) / rows);
+    g.npartials = pass_built(s.pattern, s.radius, s.dtype) ? g.pass_tiles : g.ntiles;
+}
+inline bool batch_has_passes(const BGrid &g) { return pass_built(g.pattern, g.radius, g.dtype); }
+// The buffer (0 or 1) that holds the final in.
+inline int batch_final_buf(const BGrid &g) { return ((g.iters + g.pass_sweeps) / g.pass_sweeps) & 1; }
+inline int batch_last_stage(const BGrid &g) { return g.iters + 3; }
+inline int batch_next_stage(const BGrid &g, int stage)
+{
+    if (stage < 1 || stage > g.iters + 1) return stage + 1;
+    const int next = std::min(stage + g.pass_sweeps, g.iters + 2);
+    return next == g.iters + 2 && batch_has_passes(g) ? g.iters + 3 : next;
+}
+// Tiles of a stage.
+inline int batch_stage_tiles(const BGrid &g, int stage)
+{
+    if (stage == batch_last_stage(g)) return 1;
+    return stage > 0 && batch_has_passes(g) ? g.pass_tiles : g.ntiles;
+}
 int batch_launch_round(int cls, const RoundArgs &a, unsigned blocks, hipStream_t s);
 int batch_validate_solve(const prk_solve &s);
 

@@ -43,13 +43,29 @@ template <int DT, int P, int R>
 constexpr int pass_rows()
 {
     if (P == STAR) return DT == F64 ? (R <= 5 ? 4 : 2) : DT == F32 ? (R <= 6 ? 4 : 2) : (R <= 3 ? 4 : 2);
-    if (DT == F64) return R <= 2 ? 4 : R == 3 ? 2 : 0;
+    if (DT == F64) return R <= 2 ? 4 : R <= 4 ? 2 : 0;
     if (DT == F32) return R <= 3 ? 4 : R <= 5 ? 2 : 0;
     return R <= 2 ? 2 : 0;
 }
 
 template <int DT, int P, int R>
 constexpr bool pass_ok() { return pass_rows<DT, P, R>() > 0; }
+
+template <int DT, int... I>
+constexpr bool pass_built_dtype(int pattern, int radius, std::integer_sequence<int, I...>)
+{
+    constexpr bool star[] = {pass_ok<DT, STAR, I + 1>()...}, grid[] = {pass_ok<DT, GRID, I + 1>()...};
+    return (pattern == STAR ? star : grid)[radius - 1];
+}
+
+// Whether a valid stencil has a pass kernel.
+inline bool pass_built(int pattern, int radius, int dtype)
+{
+    typedef std::make_integer_sequence<int, kMaxRadius> Radii;
+    return dtype == F64 ? pass_built_dtype<F64>(pattern, radius, Radii{})
+           : dtype == F32 ? pass_built_dtype<F32>(pattern, radius, Radii{})
+                          : pass_built_dtype<BF16>(pattern, radius, Radii{});
+}
 
 constexpr bool power_of_two(double w)
 {
@@ -61,9 +77,11 @@ constexpr bool power_of_two(double w)
 }
 
 // Tap K of one FP64 sum, in the generator's order.  A product by a power of
-// two is exact, so there the multiply and the add are one fma with the same
-// result (a product that falls below the normal range, under 2^-1022, is
-// the exception: the fma does not round it).
+// two is exact unless it falls below the normal range, so there the multiply
+// and the add are one fma with the same result.  No product falls that low:
+// a value the library refreshed (in + 1) or seeded itself is 0 or at least
+// 2^-53 in magnitude, and passes run on such values only (prk_run's first
+// sweep, which reads the caller's values, is a sweep of its own).
 template <int P, int R, int M, int V, int K>
 __device__ inline void pass_tap_f64(const double (&w)[M + 2 * R][V + 2 * R], double (&s)[M][V])
 {
@@ -176,12 +194,26 @@ __device__ inline void pass_store(__amdgpu_buffer_rsrc_t r, int col, int lo, int
     }
 }
 
+// Compensated sum of |x| (Neumaier): the lane's share of an L1 norm.
+struct NormSum {
+    double sum = 0.0, comp = 0.0;
+    __device__ inline void add(double x)
+    {
+#pragma clang fp contract(off)
+        const double a = fabs(x), t = sum + a;
+        comp += fabs(sum) >= a ? (sum - t) + a : (a - t) + sum;
+        sum = t;
+    }
+};
+
 // `sweeps` sweeps of rows [r0, r1) and the lane's V columns at cm of an
 // n x n grid: in is read, in_next gets in after `sweeps` refreshes (columns
-// below st_cols), out is updated on the interior.
+// below st_cols), out is updated on the interior.  `first`: out holds
+// nothing yet and starts from zeros, frame included (columns below st_cols).
+// `last`: adds |out| over the lane's interior points to `norm`.
 template <int DT, int P, int R, bool ALIGNED>
 __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, long long pitch, int n, int cm, int r0,
-                                 int r1, int sweeps, int st_cols)
+                                 int r1, int sweeps, int st_cols, bool first, bool last, NormSum &norm)
 {
 #pragma clang fp contract(off)
     typedef typename DTypeTraits<DT>::T T;
@@ -218,7 +250,7 @@ __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, lo
         }
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            const bool ok = o + m >= R && o + m < n - R;  // uniform
+            const bool ok = !first && o + m >= R && o + m < n - R;  // uniform
             const __amdgpu_buffer_rsrc_t r = row_rsrc(out + (long long)(ok ? o + m : 0) * pitch, ok ? row_bytes : 0u);
             Vec x;
             x.v = pass_load<DT, ALIGNED, 2>(r, cm, n);
@@ -272,6 +304,17 @@ __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, lo
         for (int m = 0; m < M; ++m) {
             const int row = o + m;
             if (row >= r1) break;  // uniform
+            const bool inner_row = row >= R && row < n - R;
+            if (last && inner_row) {
+#pragma unroll
+                for (int v = 0; v < V; ++v)
+                    if (cm + v >= R && cm + v < n - R) norm.add((double)acc_out[m][v]);
+            }
+            if (first) {
+#pragma unroll
+                for (int v = 0; v < V; ++v)
+                    acc_out[m][v] = inner_row && cm + v >= R && cm + v < n - R ? acc_out[m][v] : (C)0;
+            }
             Vec x, y;
             if constexpr (DT == F64) {
 #pragma unroll
@@ -287,7 +330,9 @@ __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, lo
                 from_f32_vec<V>(acc_out[m], y.e);
             }
             pass_store<DT, ALIGNED, 2>(row_rsrc(in_next + (long long)row * pitch, row_bytes), cm, 0, st_cols, x.v);
-            if (row >= R && row < n - R)
+            if (first)
+                pass_store<DT, ALIGNED, 2>(row_rsrc(out + (long long)row * pitch, row_bytes), cm, 0, st_cols, y.v);
+            else if (inner_row)
                 pass_store<DT, ALIGNED, 2>(row_rsrc(out + (long long)row * pitch, row_bytes), cm, R, n - R, y.v);
         }
     }
@@ -314,8 +359,9 @@ __global__ __launch_bounds__(kThreads) void pass_kernel(PassArgs a)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r0 = (band * kWavesPerBlock + wave) * a.rows;
     if (r0 >= a.n) return;
+    NormSum unused;
     pass_tile<DT, P, R, ALIGNED>(a.in, a.in_next, a.out, a.pitch, a.n, (strip * 64 + lane) * V, r0,
-                                 min(r0 + a.rows, a.n), a.sweeps, a.n);
+                                 min(r0 + a.rows, a.n), a.sweeps, a.n, false, false, unused);
 }
 
 }  // namespace prk

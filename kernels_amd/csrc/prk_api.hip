@@ -103,24 +103,6 @@ int launch_sweep(const SweepPlan &p, const void *in, void *in_next, void *out, h
     return set_error(PRK_EINVAL, "unknown dtype %d", p.dtype);
 }
 
-template <int DT>
-static bool pass_built_dtype(int pattern, int radius)
-{
-    constexpr bool ok[2][8] = {
-        {pass_ok<DT, STAR, 1>(), pass_ok<DT, STAR, 2>(), pass_ok<DT, STAR, 3>(), pass_ok<DT, STAR, 4>(),
-         pass_ok<DT, STAR, 5>(), pass_ok<DT, STAR, 6>(), pass_ok<DT, STAR, 7>(), pass_ok<DT, STAR, 8>()},
-        {pass_ok<DT, GRID, 1>(), pass_ok<DT, GRID, 2>(), pass_ok<DT, GRID, 3>(), pass_ok<DT, GRID, 4>(),
-         pass_ok<DT, GRID, 5>(), pass_ok<DT, GRID, 6>(), pass_ok<DT, GRID, 7>(), pass_ok<DT, GRID, 8>()}};
-    return ok[pattern == GRID][radius - 1];
-}
-
-bool pass_built(int pattern, int radius, int dtype)
-{
-    return dtype == F64 ? pass_built_dtype<F64>(pattern, radius)
-           : dtype == F32 ? pass_built_dtype<F32>(pattern, radius)
-                          : pass_built_dtype<BF16>(pattern, radius);
-}
-
 int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
 {
     switch (p.dtype) {

@@ -65,7 +65,6 @@ int launch_sweep_bf16(const SweepPlan &p, const void *in, void *in_next, void *o
 
 // Enqueue one pass of `sweeps` sweeps over a whole grid (pass.hpp): in_next
 // gets in after that many refreshes.  Only where pass_built.
-bool pass_built(int pattern, int radius, int dtype);
 int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
 int launch_pass_f64(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
 int launch_pass_f32(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);

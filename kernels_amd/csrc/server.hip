@@ -107,7 +107,9 @@ struct Req {
     double err_max_abs = 0, err_mean_abs = 0, err_normwise = 0;
 };
 
-constexpr int kRoundsPerWindow = 8;
+// A round is up to kServerPassSweeps sweeps of every active request, so two
+// rounds are as long as a request waits to join the running ones.
+constexpr int kRoundsPerWindow = 2;
 
 }  // namespace
 }  // namespace prk
@@ -176,10 +178,10 @@ size_t request_bytes(const prk_solve &s, BGrid &g)
     g.n = s.n;
     g.pattern = s.pattern;
     g.radius = s.radius;
-    g.iters = s.iterations;
     g.rows = std::min(s.n, 32);
     g.strips = (s.n + 64 * V - 1) / (64 * V);
     g.ntiles = g.strips * ((s.n + g.rows - 1) / g.rows);
+    batch_set_passes(g, s, kServerPassSweeps, g.rows);
     g.init_kind = s.init;
     g.seed = s.seed;
     const size_t arr = align_up((size_t)s.n * (size_t)g.pitch * dtype_size(s.dtype), 256);
@@ -372,9 +374,9 @@ int build_window(prk_server *s, long long w)
         bool any = false;
         for (size_t i = 0; i < act.size(); ++i) {
             Req *r = act[i];
-            const int last = r->g.iters + 3;
+            const int last = batch_last_stage(r->g);
             if (r->stage > last) continue;
-            const int tiles = r->stage == last ? 1 : r->g.ntiles;
+            const int tiles = batch_stage_tiles(r->g, r->stage);
             const int c = batch_class_of(r->s);
             for (int t0 = 0; t0 < tiles; t0 += kWavesPerBlock) per[c].push_back(RWork{(int)i, r->stage, t0});
             if (r->stage == last) {
@@ -382,7 +384,7 @@ int build_window(prk_server *s, long long w)
                 finishing.push_back(r);
                 finishing_grid.push_back(i);
             }
-            ++r->stage;
+            r->stage = batch_next_stage(r->g, r->stage);
             any = true;
         }
         if (!any) break;
@@ -396,7 +398,7 @@ int build_window(prk_server *s, long long w)
         std::lock_guard<std::mutex> lock(s->mu);
         std::vector<Req *> keep;
         for (Req *r : s->active)
-            if (r->stage <= r->g.iters + 3) keep.push_back(r);
+            if (r->stage <= batch_last_stage(r->g)) keep.push_back(r);
         s->active.swap(keep);
         s->inflight[slot] = finishing;
     }
@@ -717,7 +719,7 @@ int prk_server_fetch(prk_server *s, uint64_t id, int which, void *host, size_t b
     if (bytes < (size_t)r->g.n * r->g.n * es) {
         rc = set_error(PRK_EINVAL, "host buffer too small");
     } else {
-        const void *src = which == 0 ? r->g.out : ((r->s.iterations + 1) % 2 ? r->g.buf1 : r->g.buf0);
+        const void *src = which == 0 ? r->g.out : (batch_final_buf(r->g) ? r->g.buf1 : r->g.buf0);
         rc = check_hip(hipMemcpy2D(host, (size_t)r->g.n * es, src, (size_t)r->g.pitch * es, (size_t)r->g.n * es,
                                    (size_t)r->g.n, hipMemcpyDeviceToHost),
                        "server fetch");

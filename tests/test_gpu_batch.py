@@ -333,3 +333,23 @@ def test_random_mix_bitwise(gpu, oracle, rows):
         assert abs(norms[i] - norm) <= 1e-13 * abs(norm) + 1e-300, (s, norms[i], norm)
     b.close()
 
+
+
+def test_solves_of_more_than_one_pass(gpu, oracle):
+    # 64 sweeps are one pass, 65 two of 33 and 32, 130 three: the buffer that
+    # ends up with in, the first pass's zeroed out (frame included) and the
+    # last one's norm partials, beside solves that need one pass and one
+    # without a pass kernel
+    specs = [(0, 2, F64, 130, 64, 1, 71), (1, 3, F32, 77, 129, 1, 72), (0, 1, BF16, 530, 63, 1, 73),
+             (1, 4, F64, 41, 70, 1, 74), (1, 2, F32, 260, 0, 1, 75), (1, 6, F32, 20, 5, 1, 76)]
+    b = Batch(specs)
+    for _ in range(2):
+        b.run()
+        norms = b.wait()
+    for i, s in enumerate(specs):
+        print(f"solve {i}: {s}", flush=True)
+        out, fin, norm = ref_solve(oracle, s)
+        assert np.array_equal(b.output(i, 0).view(np.uint8), out.view(np.uint8)), s
+        assert np.array_equal(b.output(i, 1).view(np.uint8), fin.view(np.uint8)), s
+        assert abs(norms[i] - norm) <= 1e-13 * abs(norm), s
+    b.close()
