@@ -73,9 +73,8 @@ int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const
     const size_t es = dtype_size(dtype);
     if ((unsigned long long)pitch * es >= (1ull << 31))
         return set_error(PRK_EINVAL, "row of %lld elements exceeds 2 GiB", pitch);
-    const bool aligned = ((uintptr_t)in % 16 == 0) && ((uintptr_t)out % 16 == 0) &&
-                         (!in_next || (uintptr_t)in_next % 16 == 0) && ((pitch * es) % 16 == 0);
-    const int V = vec_width(dtype);
+    const unsigned long long ptrs =
+        (uintptr_t)in | (uintptr_t)out | (uintptr_t)in_next | (unsigned long long)pitch * es;  // the bits every row's address has
     plan->dtype = dtype;
     plan->pattern = pattern;
     plan->radius = radius;
@@ -83,7 +82,10 @@ int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const
     plan->span = whole_grid(n);
     plan->pitch = pitch;
     plan->pad_writable = false;
-    plan->mode = !aligned ? MODE_ELEM : (n % V == 0 ? MODE_VEC : MODE_VEC_LD);
+    plan->mode = ptrs % 4 != 0                ? MODE_ELEM
+                 : ptrs % 16 != 0             ? MODE_DWORD
+                 : n % vec_width(dtype) != 0 ? MODE_RAGGED
+                                              : MODE_VEC;
     const prk_tuning t = choose_tuning(pattern, radius, dtype, n);
     plan->variant = g_variant_override >= 0 ? g_variant_override : t.variant;
     plan->order = g_order >= 0 ? g_order : t.order;
@@ -680,7 +682,7 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     // asks for the sweep kernel itself: one sweep per pass then.
     const bool overridden = g_rows_per_wave > 0 || g_variant_override >= 0 || g_order >= 0 || g_wgs_per_cu >= 0;
     int passes = iterations;
-    if (!overridden && pass_built(pattern, radius, dtype)) {
+    if (!overridden && pass_built(pattern, radius, dtype) && (p.mode != MODE_ELEM || dtype == BF16)) {
         passes = (iterations + kMaxPassSweeps - 1) / kMaxPassSweeps;
         passes += (passes ^ iterations) & 1;
     }

@@ -21,7 +21,7 @@ struct SweepPlan {
     RowSpan span;                   // rows read and written (prk_common.hpp)
     long long pitch;
     int rows_per_wave;
-    int mode;           // MODE_ELEM / MODE_VEC / MODE_VEC_LD (sweep.hpp)
+    int mode;           // MODE_* (sweep.hpp)
     int variant;        // pipeline depth / cache policy of the fused vector sweep
     bool pad_writable;  // columns n..pitch-1 may be overwritten
     int order;          // workgroup -> tile order (sweep.hpp tile_of)

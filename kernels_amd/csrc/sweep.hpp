@@ -691,9 +691,59 @@ __device__ inline void bstore_elem(__amdgpu_buffer_rsrc_t r, unsigned off, T v)
 // Access modes of the sweep.
 //   MODE_VEC    rows 16-byte aligned and every written vector whole: n % V == 0,
 //               or the caller lets columns n..pitch-1 be overwritten.
-//   MODE_VEC_LD 16-byte vector loads, element stores (aligned rows, ragged n).
-//   MODE_ELEM   element loads and stores (rows not 16-byte aligned).
-enum { MODE_ELEM = 0, MODE_VEC = 1, MODE_VEC_LD = 2 };
+//   MODE_RAGGED rows 16-byte aligned, a vector straddles column n: 16-byte
+//               loads and stores, that vector's elements stored one by one.
+//               (A mode of its own: the test for such a wave in the row loop
+//               cost the MODE_VEC sweeps 1-12 % on MI355X.)
+//   MODE_DWORD  rows 4-byte aligned: the same (a buffer access of 16 bytes
+//               needs no more), but a row's last vector may run past the row.
+//               The bytes behind it are the next row's, so it is loaded whole
+//               there too; only the array's last row is read by element.
+//   MODE_ELEM   element loads and stores (BF16 rows on odd elements).
+// Measured on MI355X, element accesses -> these: fused sweeps at n=9999, rows
+// on 128 bytes, FP32 star R=1 421 -> 274 us (n=10000: 274), FP64 star R=2
+// 640 -> 536, BF16 grid R=3 331 -> 167; at n=4001, pitch 4001, FP64 star R=2
+// 119 -> 96 us, FP32 71 -> 55.
+enum { MODE_ELEM = 0, MODE_VEC = 1, MODE_DWORD = 2, MODE_RAGGED = 3 };
+
+// One row's V elements at byte offset off (kOOB: none).  `end`: the row is
+// the array's last (MODE_DWORD only).
+template <typename T, int V, int MODE, int AUX>
+__device__ inline u32x4 load_row_vec(__amdgpu_buffer_rsrc_t r, unsigned off, bool end)
+{
+    if (MODE == MODE_VEC || MODE == MODE_RAGGED || (MODE == MODE_DWORD && !end)) return bload16<AUX>(r, off);
+    union { u32x4 v; T e[V]; } x;
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        x.e[v] = bload_elem<T, AUX>(r, off != kOOB ? off + (unsigned)(v * sizeof(T)) : kOOB);
+    return x.v;
+}
+
+// Byte range of the resource a row is loaded through.
+template <int MODE>
+__device__ inline unsigned row_load_bytes(unsigned row_bytes, bool end)
+{
+    return MODE == MODE_DWORD && !end ? min(row_bytes + 16u, kOOB) : row_bytes;
+}
+
+// One vector of in_next at byte offset off (kOOB: none); `ragged`: the wave
+// holds the vector that straddles column n.
+template <typename T, int V, int MODE, int AUX>
+__device__ inline void store_next_vec(__amdgpu_buffer_rsrc_t r, unsigned off, int cm, int n, bool ragged,
+                                      const u32x4 &val)
+{
+    if (MODE == MODE_VEC || (MODE != MODE_ELEM && !ragged)) {
+        bstore16<AUX>(r, off, val);
+        return;
+    }
+    const bool whole = MODE != MODE_ELEM && cm + V <= n;
+    if constexpr (MODE != MODE_ELEM) bstore16<AUX>(r, whole ? off : kOOB, val);
+    union { u32x4 v; T e[V]; } x;
+    x.v = val;
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        bstore_elem<T, AUX>(r, whole || off == kOOB || cm + v >= n ? kOOB : off + (unsigned)(v * sizeof(T)), x.e[v]);
+}
 
 // One wavefront's tile: columns [c0, c0+64V) of rows [r0, r1) of an array of
 // sp.nrows rows and n columns.  ring points at this wave's (2R+1) x LR
@@ -786,7 +836,7 @@ __device__ inline void flush_edge_stash(const u32x4 *stash, T *out, long long pi
         const int col = side == 0 ? R : n - R;  // first interior / first right frame column
         const int cb = col - col % V;           // the vector holding it
         if (col % V == 0 || cb < c0 || cb >= c0 + sw) continue;
-        if (side == 1 && cb == cb_left) continue;  // one vector holds both boundaries
+        if (side == 1 && R % V != 0 && cb == cb_left) continue;  // one vector holds both boundaries
         if (lane < nout) {
             union { u32x4 v; T e[V]; } x;
             x.v = stash[2 * lane + side];
@@ -832,7 +882,7 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = FRAME == FRAME_KEEP && MODE == MODE_VEC && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = FRAME == FRAME_KEEP && MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -842,6 +892,8 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
     // caller allows the padding to be written.
     const unsigned ld_bytes = (unsigned)(pitch * ES);
     const unsigned st_bytes = pad_writable ? ld_bytes : (unsigned)(n * ES);
+    // wave-uniform: the strip holds a vector with columns on both sides of n
+    const bool ragged = !pad_writable && n % V != 0 && c0 + SweepGeom<DT, R>::SW > n;
 
     const int cm = c0 + lane * V;  // first column of this lane's main vector
     // Halo vector of this lane (lanes 0..NH-1 left, NH..2NH-1 right); other
@@ -859,22 +911,16 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
     auto issue = [&](RowRegs<T, V> &r, int ri) {
         const bool row_ok = ri < hi;
         const int rr = row_ok ? ri : lo;
-        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, ld_bytes);
+        const bool end = rr + 1 == sp.nrows;
+        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, row_load_bytes<MODE>(ld_bytes, end));
         const int o = ri - R;
         const bool out_ok = o >= olo && o < ohi;
-        const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, ld_bytes);
-        if constexpr (MODE != MODE_ELEM) {
-            r.main.v = bload16<AUX_IN>(rin, row_ok ? off_main : kOOB);
-            r.halo.v = bload16<AUX_IN>(rin, row_ok ? off_halo : kOOB);
-            r.outv.v = bload16<AUX_OUT_LD>(rout, out_ok ? off_main : kOOB);
-        } else {
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                r.main.e[v] = bload_elem<T, AUX_IN>(rin, row_ok ? off_main + v * ES : kOOB);
-                r.halo.e[v] = bload_elem<T, AUX_IN>(rin, (row_ok && off_halo != kOOB) ? off_halo + v * ES : kOOB);
-                r.outv.e[v] = bload_elem<T, AUX_OUT_LD>(rout, out_ok ? off_main + v * ES : kOOB);
-            }
-        }
+        // rows of out that are read are interior: never the last
+        const __amdgpu_buffer_rsrc_t rout =
+            row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, row_load_bytes<MODE>(ld_bytes, !out_ok));
+        r.main.v = load_row_vec<T, V, MODE, AUX_IN>(rin, row_ok ? off_main : kOOB, end);
+        r.halo.v = load_row_vec<T, V, MODE, AUX_IN>(rin, row_ok ? off_halo : kOOB, end);
+        r.outv.v = load_row_vec<T, V, MODE, AUX_OUT_LD>(rout, out_ok ? off_main : kOOB, false);
     };
 
 #pragma unroll
@@ -898,13 +944,7 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
                     row_rsrc(in_next + (long long)(nx_ok ? ri : r0) * pitch, st_bytes);
                 union { u32x4 v; T e[V]; } nx;
                 plus_one<DT, V>(cur.main.e, nx.e);
-                if constexpr (MODE == MODE_VEC) {
-                    bstore16<AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, nx.v);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        bstore_elem<T, AUX_STREAM>(rnx, nx_ok ? off_main + v * ES : kOOB, nx.e[v]);
-                }
+                store_next_vec<T, V, MODE, AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, cm, n, ragged, nx.v);
             }
 
             // LDS writes of this wave land before its reads (in-order per
@@ -930,13 +970,13 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
                 union { u32x4 v; T e[V]; } res;
                 compute_points<DT, P, R, V, HP>(rows, cur.outv.e, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE == MODE_VEC && FRAME == FRAME_REWRITE) {
+                if constexpr (MODE != MODE_ELEM && FRAME == FRAME_REWRITE) {
                     unsigned off[V];
                     out_offsets<V, ES>(c0, n, R, off);
 #pragma unroll
                     for (int v = 0; v < V; ++v) res.e[v] = off[v] != kOOB ? res.e[v] : cur.outv.e[v];
                     bstore16<AUX_STREAM>(rout, off_main, res.v);
-                } else if constexpr (MODE == MODE_VEC) {
+                } else if constexpr (MODE != MODE_ELEM) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {
@@ -993,7 +1033,7 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = MODE == MODE_VEC && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1001,6 +1041,8 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
     T *out = (T *)out_;
     const unsigned ld_bytes = (unsigned)(pitch * ES);
     const unsigned st_bytes = pad_writable ? ld_bytes : (unsigned)(n * ES);
+    // wave-uniform: the strip holds a vector with columns on both sides of n
+    const bool ragged = !pad_writable && n % V != 0 && c0 + SweepGeom<DT, R>::SW > n;
 
     const int cm = c0 + lane * V;
     const int ch = lane < NH ? c0 - HP + lane * V : c0 + G::SW + (lane - NH) * V;
@@ -1018,22 +1060,16 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
     auto issue = [&](Vec &m, Side &sd, int ri) {
         const bool row_ok = ri < hi;
         const int rr = row_ok ? ri : lo;
-        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, ld_bytes);
+        const bool end = rr + 1 == sp.nrows;
+        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, row_load_bytes<MODE>(ld_bytes, end));
         const int o = ri - R;
         const bool out_ok = o >= olo && o < ohi;
-        const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, ld_bytes);
-        if constexpr (MODE != MODE_ELEM) {
-            m.v = bload16<0>(rin, row_ok ? off_main : kOOB);
-            sd.halo.v = bload16<0>(rin, row_ok ? off_halo : kOOB);
-            sd.outv.v = bload16<AUX_STREAM>(rout, out_ok ? off_main : kOOB);
-        } else {
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                m.e[v] = bload_elem<T, 0>(rin, row_ok ? off_main + v * ES : kOOB);
-                sd.halo.e[v] = bload_elem<T, 0>(rin, (row_ok && off_halo != kOOB) ? off_halo + v * ES : kOOB);
-                sd.outv.e[v] = bload_elem<T, AUX_STREAM>(rout, out_ok ? off_main + v * ES : kOOB);
-            }
-        }
+        // rows of out that are read are interior: never the last
+        const __amdgpu_buffer_rsrc_t rout =
+            row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, row_load_bytes<MODE>(ld_bytes, !out_ok));
+        m.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_main : kOOB, end);
+        sd.halo.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_halo : kOOB, end);
+        sd.outv.v = load_row_vec<T, V, MODE, AUX_STREAM>(rout, out_ok ? off_main : kOOB, false);
     };
 
 #pragma unroll
@@ -1059,13 +1095,7 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
                     row_rsrc(in_next + (long long)(nx_ok ? ri : r0) * pitch, st_bytes);
                 Vec nx;
                 plus_one<DT, V>(cur.e, nx.e);
-                if constexpr (MODE == MODE_VEC) {
-                    bstore16<AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, nx.v);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        bstore_elem<T, AUX_STREAM>(rnx, nx_ok ? off_main + v * ES : kOOB, nx.e[v]);
-                }
+                store_next_vec<T, V, MODE, AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, cm, n, ragged, nx.v);
             }
 
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1087,7 +1117,7 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
                 Vec res;
                 star_points<DT, R, V, HP>(&ring[cs][HP + lane * V], col, sd.outv.e, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE == MODE_VEC) {
+                if constexpr (MODE != MODE_ELEM) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {
@@ -1250,7 +1280,7 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = MODE == MODE_VEC && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1258,6 +1288,8 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
     T *out = (T *)out_;
     const unsigned ld_bytes = (unsigned)(pitch * ES);
     const unsigned st_bytes = pad_writable ? ld_bytes : (unsigned)(n * ES);
+    // wave-uniform: the strip holds a vector with columns on both sides of n
+    const bool ragged = !pad_writable && n % V != 0 && c0 + SweepGeom<DT, R>::SW > n;
 
     const int cm = c0 + lane * V;
     // halo vectors: lane 0 the V columns left of the strip, lane 1 the V
@@ -1273,22 +1305,16 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
     auto issue = [&](RowRegs<T, V> &r, int ri) {
         const bool row_ok = ri < hi;
         const int rr = row_ok ? ri : lo;
-        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, ld_bytes);
+        const bool end = rr + 1 == sp.nrows;
+        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, row_load_bytes<MODE>(ld_bytes, end));
         const int o = ri - R;
         const bool out_ok = o >= olo && o < ohi;
-        const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, ld_bytes);
-        if constexpr (MODE != MODE_ELEM) {
-            r.main.v = bload16<0>(rin, row_ok ? off_main : kOOB);
-            r.halo.v = bload16<0>(rin, row_ok ? off_halo : kOOB);
-            r.outv.v = bload16<AUX_STREAM>(rout, out_ok ? off_main : kOOB);
-        } else {
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                r.main.e[v] = bload_elem<T, 0>(rin, row_ok ? off_main + v * ES : kOOB);
-                r.halo.e[v] = bload_elem<T, 0>(rin, (row_ok && off_halo != kOOB) ? off_halo + v * ES : kOOB);
-                r.outv.e[v] = bload_elem<T, AUX_STREAM>(rout, out_ok ? off_main + v * ES : kOOB);
-            }
-        }
+        // rows of out that are read are interior: never the last
+        const __amdgpu_buffer_rsrc_t rout =
+            row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, row_load_bytes<MODE>(ld_bytes, !out_ok));
+        r.main.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_main : kOOB, end);
+        r.halo.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_halo : kOOB, end);
+        r.outv.v = load_row_vec<T, V, MODE, AUX_STREAM>(rout, out_ok ? off_main : kOOB, false);
     };
 
 #pragma unroll
@@ -1308,13 +1334,7 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
                     row_rsrc(in_next + (long long)(nx_ok ? ri : r0) * pitch, st_bytes);
                 union { u32x4 v; T e[V]; } nx;
                 plus_one<DT, V>(cur.main.e, nx.e);
-                if constexpr (MODE == MODE_VEC) {
-                    bstore16<AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, nx.v);
-                } else {
-#pragma unroll
-                    for (int v = 0; v < V; ++v)
-                        bstore_elem<T, AUX_STREAM>(rnx, nx_ok ? off_main + v * ES : kOOB, nx.e[v]);
-                }
+                store_next_vec<T, V, MODE, AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, cm, n, ragged, nx.v);
             }
 
             // lane 63's right neighbours: the right halo vector, loaded by lane 1
@@ -1333,7 +1353,7 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
                 union { u32x4 v; T e[V]; } res;
                 from_f32_vec<V>(f, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE == MODE_VEC) {
+                if constexpr (MODE != MODE_ELEM) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {

@@ -54,7 +54,7 @@ int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hip
     // kStashRows rows of out from one resource, which must stay below the
     // out-of-range offset.
     a.stash = 0;
-    if (!RW && MODE == MODE_VEC &&
+    if (!RW && MODE != MODE_ELEM &&
         (long long)kStashRows * p.pitch * (long long)sizeof(typename G::T) < (long long)kOOB) {
         if (dyn >= kStashBytes) {
             a.stash = 1;
@@ -74,10 +74,10 @@ int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hip
     return check_hip(hipGetLastError(), "sweep launch");
 }
 
-// The fused, whole-vector sweep is the hot path: it is instantiated for
+// The fused sweep of aligned rows is the hot path: it is instantiated for
 // every pipeline depth / cache policy the tuner chooses from (radii beyond
 // the reference's 5: one, two rows in flight with non-temporal stores).  The
-// other forms use the default.  Four rows in flight (variant 8) made FP64
+// other forms have one variant each.  Four rows in flight (variant 8) made FP64
 // star R=2 at n=30000 1.3-1.8 % faster than three at 6- and 8-row blocks
 // on MI355X (alternating runs on one box), and slower at 12 and 16 rows.
 template <int DT, int P, int R>
@@ -106,11 +106,14 @@ int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipS
         }
     }
     if (fuse) {
-        if (p.mode == MODE_VEC_LD) return launch_one<DT, P, R, true, MODE_VEC_LD, kPrefetch, 0>(p, in, in_next, out, s);
+        constexpr int PF = R > kRefMaxRadius ? 2 : 3;
+        if (p.mode == MODE_RAGGED) return launch_one<DT, P, R, true, MODE_RAGGED, PF, 1>(p, in, in_next, out, s);
+        if (p.mode == MODE_DWORD) return launch_one<DT, P, R, true, MODE_DWORD, PF, 1>(p, in, in_next, out, s);
         return launch_one<DT, P, R, true, MODE_ELEM, kPrefetch, 0>(p, in, in_next, out, s);
     }
     if (p.mode == MODE_VEC) return launch_one<DT, P, R, false, MODE_VEC, kPrefetch, 0>(p, in, in_next, out, s);
-    if (p.mode == MODE_VEC_LD) return launch_one<DT, P, R, false, MODE_VEC_LD, kPrefetch, 0>(p, in, in_next, out, s);
+    if (p.mode == MODE_RAGGED) return launch_one<DT, P, R, false, MODE_RAGGED, kPrefetch, 0>(p, in, in_next, out, s);
+    if (p.mode == MODE_DWORD) return launch_one<DT, P, R, false, MODE_DWORD, kPrefetch, 0>(p, in, in_next, out, s);
     return launch_one<DT, P, R, false, MODE_ELEM, kPrefetch, 0>(p, in, in_next, out, s);
 }
 
@@ -160,7 +163,7 @@ int launch_pass_pr(const SweepPlan &p, int sweeps, const void *in, void *in_next
         a.sweeps = sweeps;
         const int per_block = a.rows * kWavesPerBlock;
         const unsigned blocks = (unsigned)a.nstrips * (unsigned)((p.n + per_block - 1) / per_block);
-        if (p.mode != MODE_ELEM)
+        if (p.mode == MODE_VEC || p.mode == MODE_RAGGED)
             hipLaunchKernelGGL((pass_kernel<DT, P, R, true>), dim3(blocks), dim3(kThreads), 0, s, a);
         else
             hipLaunchKernelGGL((pass_kernel<DT, P, R, false>), dim3(blocks), dim3(kThreads), 0, s, a);

@@ -452,3 +452,35 @@ def test_edge_stash_paths(gpu, oracle, dtype, pattern, radius, n):
     finally:
         K.check(L.prk_set_sweep_variant(-1)); K.check(L.prk_set_rows_per_wave(0))
         K.check(L.prk_set_sweep_order(-1, -1))
+
+
+@pytest.mark.parametrize("pitch_off", [0, 1, 2])
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("pattern,radius", [(0, 1), (0, 2), (1, 3), (0, 6), (1, 7)])
+def test_ragged_and_misaligned_rows_bitwise(gpu, oracle, pattern, radius, dtype, pitch_off):
+    # n on either side of a whole number of vectors and strips, down to the
+    # smallest grid (one vector holding both frame boundaries), rows on 16
+    # bytes (pitch_off 0) or on elements only: one fused sweep and one
+    # unfused one against the oracle's two sweeps.  Columns past n keep what
+    # they held; with pitch n the array's last row ends the allocation.
+    V = {0: 2, 1: 4, 2: 8}[dtype]
+    for n in sorted({2 * radius + 1, 2 * radius + 2, 64 * V - 1, 64 * V + 1, 64 * V + V + 3}):
+        pitch = (n + V - 1) // V * V if pitch_off == 0 else n if pitch_off == 1 else n + (2 if n % 2 == 0 else 1)
+        print(f"p{pattern} r{radius} d{dtype} n={n} pitch={pitch}", flush=True)
+        base = [torch.full((n, pitch), 3.0, dtype=K.torch_dtype(dtype), device=gpu) for _ in range(3)]
+        b0, b1, out = (b[:, :n] for b in base)
+        K.init(K.INIT_SEEDED, n, dtype, b0, out)
+        K.sweep(pattern, radius, dtype, b0, b1, out)
+        K.stencil_ex(pattern, radius, dtype, b1, out)
+        if dtype == K.F64:
+            ref_out, _ = oracle.run(pattern, radius, n, 32, 1, 1, n)
+            _, ref_in = oracle.run(pattern, radius, n, 32, 0, 1, n)
+        else:
+            ref_out, _ = oracle.run_lp(dtype, pattern, radius, n, 1, 1, n)
+            _, ref_in = oracle.run_lp(dtype, pattern, radius, n, 0, 1, n)
+        view = {0: torch.int64, 1: torch.int32, 2: torch.int16}[dtype]
+        for got, ref in ((out, ref_out), (b1, ref_in)):
+            g = got.contiguous().view(view).cpu().numpy()
+            assert np.array_equal(g, ref.view(g.dtype)), (n, pitch)
+        for b in base:
+            assert bool((b[:, n:] == 3.0).all()), (n, pitch)
