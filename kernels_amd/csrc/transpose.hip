@@ -2,19 +2,21 @@
 // (Cxx11/transpose.cc:118-131; the HIP driver's transposeNoBankConflict,
 // Cxx11/transpose-hip.cc:64-87), both matrices order x order FP64, row-major.
 //
-// Mapping.  A workgroup (four waves) owns one tile of A, 64 rows x 128
-// columns by default.  It reads the tile's rows with 16-byte buffer loads
-// (one 1 KiB row segment per wave and pass), writes A + 1 back to the same
-// addresses, and parks the tile in LDS (rows padded by one element so that
-// reading a column spreads over the banks).  After a barrier it reads the
-// tile's columns from LDS and adds them to the matching rows of B (16-byte
-// loads and stores again, 512-byte row segments).  Every
-// element of A and B is read once and written once: 32 bytes per element,
-// the algorithmic traffic of the reference's Rate (4 * 8 * order^2 bytes).
-// All eight loads of a phase are issued before the first is consumed.
+// Mapping.  A workgroup owns one tile of A.  It reads the tile's rows of A
+// with 16-byte buffer loads, all of them issued before the first is used,
+// writes A + 1 back to the same addresses, and parks the tile in LDS (rows
+// padded by one element so that reading a column spreads over the banks).
+// Then it issues the loads of the matching rows of B, waits for the others'
+// share of the tile, adds the tile's columns to B and stores it.  Every element of A and B is read once
+// and written once: 32 bytes per element, the algorithmic traffic of the
+// reference's Rate (4 * 8 * order^2 bytes).  What bounds it is HBM, at the
+// rate the tiles' short row segments reach (launch_transpose).
 // Edges: rows and columns beyond `order` are out-of-range buffer offsets
-// (reads give 0, writes are dropped).  Odd orders use 64 x 64 tiles and
-// 8-byte accesses.
+// (reads give 0, writes are dropped).  Where order is odd, rows start on
+// 8-byte boundaries, which the 16-byte accesses take as they are; the tiles
+// that hold a row's last column, whose vector would run past the row, move
+// single elements.  Large matrices with such rows have a kernel of 8-byte
+// accesses.
 //
 // Values stay integers below 2^53 (order^2 * (iterations + 1) plus the
 // added ones), so every sum is exact and results equal the reference's bit
@@ -30,9 +32,6 @@
 
 namespace prk {
 namespace {
-
-constexpr int kT = 64;          // tile edge (the odd-order kernel, and the tile-count unit)
-constexpr int kTThreads = 256;  // four waves
 
 struct TransposeArgs {
     double *A;
@@ -62,83 +61,128 @@ __device__ inline void tile_of_transpose(const TransposeArgs &a, int b, int &tr,
     }
 }
 
-// One TR x TC tile of A (TR rows, TC columns): VE doubles per lane access
-// (2: 16 bytes; 1: odd orders).  NT: non-temporal stores.
-template <int TR, int TC, int VE, int NT, int NTH>
+// Two neighbouring elements; SPLIT: as single ones, without the second
+// where `last` (offsets of kOOB and above, up to the 95 MB a tile spans, are
+// out of range).
+template <int AUX, bool SPLIT>
+__device__ inline u32x4 load2(__amdgpu_buffer_rsrc_t r, unsigned off, bool last)
+{
+    if constexpr (!SPLIT) return bload16<AUX>(r, off);
+    union { u32x4 v; double d[2]; } x;
+    x.d[0] = bload_elem<double, AUX>(r, off);
+    x.d[1] = bload_elem<double, AUX>(r, last ? kOOB : off + 8u);
+    return x.v;
+}
+
+template <int AUX, bool SPLIT>
+__device__ inline void store2(__amdgpu_buffer_rsrc_t r, unsigned off, bool last, const u32x4 &v)
+{
+    if constexpr (!SPLIT) {
+        bstore16<AUX>(r, off, v);
+    } else {
+        union { u32x4 v; double d[2]; } x;
+        x.v = v;
+        bstore_elem<double, AUX>(r, off, x.d[0]);
+        bstore_elem<double, AUX>(r, last ? kOOB : off + 8u, x.d[1]);
+    }
+}
+
+// One TR x TC tile of A (TR rows, TC columns) on NTH threads.  NT: loads and
+// stores marked non-temporal.
+template <int TR, int TC, int NTH, bool NT, bool SPLIT>
+__device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, double (*tile)[TC + 1])
+{
+    constexpr int LPR1 = TC / 2, RPP1 = NTH / LPR1, NP1 = TR / RPP1;  // A rows
+    constexpr int LPR2 = TR / 2, RPP2 = NTH / LPR2, NP2 = TC / RPP2;  // B rows
+    static_assert(NP1 >= 1 && NP2 >= 1 && RPP1 * NP1 == TR && RPP2 * NP2 == TC, "tile shape");
+    constexpr int AUX = NT ? 2 : 0;
+    const int order = a.order;
+    const unsigned row_bytes = (unsigned)order * 8u;
+    union V { u32x4 v; double d[2]; };
+    // One resource per matrix, the rows of the tile (at most 256 rows of
+    // 46340 elements: 95 MB), so that it is the same in every lane; rows past
+    // the last lie beyond its range, columns past the last are moved there.
+    const __amdgpu_buffer_rsrc_t ra =
+        row_rsrc(a.A + (long long)tr * TR * order, (unsigned)min(TR, order - tr * TR) * row_bytes);
+    const __amdgpu_buffer_rsrc_t rb =
+        row_rsrc(a.B + (long long)tc * TC * order, (unsigned)min(TC, order - tc * TC) * row_bytes);
+    // this thread's elements: of A, rows tr*TR + p*RPP1 + ar, columns ac and
+    // ac + 1 of the tile; of B, rows tc*TC + p*RPP2 + br, columns bc, bc + 1
+    const int ar = threadIdx.x / LPR1, ac = (threadIdx.x - ar * LPR1) * 2;
+    const int br = threadIdx.x / LPR2, bc = (threadIdx.x - br * LPR2) * 2;
+    const unsigned off_a = tc * TC + ac < order ? ar * row_bytes + (unsigned)(tc * TC + ac) * 8u : kOOB;
+    const unsigned off_b = tr * TR + bc < order ? br * row_bytes + (unsigned)(tr * TR + bc) * 8u : kOOB;
+    const unsigned step_a = RPP1 * row_bytes, step_b = RPP2 * row_bytes;
+    // the last column's second element would be the next row's first
+    const bool last_a = tc * TC + ac + 1 >= order, last_b = tr * TR + bc + 1 >= order;
+
+    V x[NP1], y[NP2];
+#pragma unroll
+    for (int p = 0; p < NP1; ++p) x[p].v = load2<AUX, SPLIT>(ra, off_a + p * step_a, last_a);
+#pragma unroll
+    for (int p = 0; p < NP1; ++p) {
+        V z;
+        z.d[0] = x[p].d[0] + 1.0;
+        z.d[1] = x[p].d[1] + 1.0;
+        tile[p * RPP1 + ar][ac] = x[p].d[0];
+        tile[p * RPP1 + ar][ac + 1] = x[p].d[1];
+        store2<AUX, SPLIT>(ra, off_a + p * step_a, last_a, z.v);
+    }
+#pragma unroll
+    for (int p = 0; p < NP2; ++p) y[p].v = load2<AUX, SPLIT>(rb, off_b + p * step_b, last_b);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < NP2; ++p) {
+        y[p].d[0] = y[p].d[0] + tile[bc][p * RPP2 + br];
+        y[p].d[1] = y[p].d[1] + tile[bc + 1][p * RPP2 + br];
+        store2<AUX, SPLIT>(rb, off_b + p * step_b, last_b, y[p].v);
+    }
+}
+
+// ODD: order is odd; the tiles that hold the last column of A or B split
+// their vectors.
+template <int TR, int TC, int NTH, bool NT, bool ODD>
 __global__ __launch_bounds__(NTH) void transpose_kernel(TransposeArgs a)
 {
-    constexpr int LPR1 = TC / VE, RPP1 = NTH / LPR1, NP1 = TR / RPP1;  // A rows
-    constexpr int LPR2 = TR / VE, RPP2 = NTH / LPR2, NP2 = TC / RPP2;  // B rows
-    static_assert(NP1 >= 1 && NP2 >= 1 && RPP1 * NP1 == TR && RPP2 * NP2 == TC, "tile shape");
-    constexpr int AUX_ST = NT ? 2 : 0;
     __shared__ double tile[TR][TC + 1];
+    int tr, tc;
+    tile_of_transpose(a, blockIdx.x, tr, tc);
+    if (ODD && ((tc + 1) * TC > a.order || (tr + 1) * TR > a.order))
+        transpose_tile<TR, TC, NTH, NT, true>(a, tr, tc, tile);
+    else
+        transpose_tile<TR, TC, NTH, NT, false>(a, tr, tc, tile);
+}
 
+// One 64 x 64 tile of A in 8-byte accesses, non-temporal stores.
+__global__ __launch_bounds__(256) void transpose_kernel_8b(TransposeArgs a)
+{
+    constexpr int T = 64, RPP = 4, NP = T / RPP;  // four rows at a time
+    __shared__ double tile[T][T + 1];
     int tr, tc;
     tile_of_transpose(a, blockIdx.x, tr, tc);
     const int order = a.order;
     const unsigned row_bytes = (unsigned)order * 8u;
-    union V { u32x4 v; double d[2]; };
-
-    // phase 1: A tile rows -> registers -> (A + 1, LDS)
-    {
-        const int lr = threadIdx.x / LPR1, lc = (threadIdx.x - lr * LPR1) * VE;
-        const int c = tc * TC + lc;
-        const unsigned off = c < order ? (unsigned)c * 8u : kOOB;
-        V x[NP1];
-        __amdgpu_buffer_rsrc_t rs[NP1];
+    const __amdgpu_buffer_rsrc_t ra =
+        row_rsrc(a.A + (long long)tr * T * order, (unsigned)min(T, order - tr * T) * row_bytes);
+    const __amdgpu_buffer_rsrc_t rb =
+        row_rsrc(a.B + (long long)tc * T * order, (unsigned)min(T, order - tc * T) * row_bytes);
+    const int r = threadIdx.x / T, c = threadIdx.x % T;
+    const unsigned step = RPP * row_bytes;
+    const unsigned off_a = tc * T + c < order ? r * row_bytes + (unsigned)(tc * T + c) * 8u : kOOB;
+    const unsigned off_b = tr * T + c < order ? r * row_bytes + (unsigned)(tr * T + c) * 8u : kOOB;
+    double x[NP];
 #pragma unroll
-        for (int p = 0; p < NP1; ++p) {
-            const int r = tr * TR + p * RPP1 + lr;
-            const bool ok = r < order;
-            rs[p] = row_rsrc(a.A + (long long)(ok ? r : 0) * order, ok ? row_bytes : 0u);
-            if constexpr (VE == 2)
-                x[p].v = bload16<0>(rs[p], off);
-            else
-                x[p].d[0] = bload_elem<double, 0>(rs[p], off);
-        }
+    for (int p = 0; p < NP; ++p) x[p] = bload_elem<double, 0>(ra, off_a + p * step);
 #pragma unroll
-        for (int p = 0; p < NP1; ++p) {
-            V y;
-#pragma unroll
-            for (int e = 0; e < VE; ++e) {
-                y.d[e] = x[p].d[e] + 1.0;
-                tile[p * RPP1 + lr][lc + e] = x[p].d[e];
-            }
-            if constexpr (VE == 2)
-                bstore16<AUX_ST>(rs[p], off, y.v);
-            else
-                bstore_elem<double, AUX_ST>(rs[p], off, y.d[0]);
-        }
+    for (int p = 0; p < NP; ++p) {
+        tile[p * RPP + r][c] = x[p];
+        bstore_elem<double, 2>(ra, off_a + p * step, x[p] + 1.0);
     }
     __syncthreads();
-    // phase 2: B rows tc*TC + q, columns tr*TR + lc: B[y][x] += A[x][y]
-    {
-        const int lr = threadIdx.x / LPR2, lc = (threadIdx.x - lr * LPR2) * VE;
-        const int c = tr * TR + lc;
-        const unsigned off = c < order ? (unsigned)c * 8u : kOOB;
-        V b[NP2];
-        __amdgpu_buffer_rsrc_t rs[NP2];
 #pragma unroll
-        for (int p = 0; p < NP2; ++p) {
-            const int y = tc * TC + p * RPP2 + lr;
-            const bool ok = y < order;
-            rs[p] = row_rsrc(a.B + (long long)(ok ? y : 0) * order, ok ? row_bytes : 0u);
-            if constexpr (VE == 2)
-                b[p].v = bload16<0>(rs[p], off);
-            else
-                b[p].d[0] = bload_elem<double, 0>(rs[p], off);
-        }
+    for (int p = 0; p < NP; ++p) x[p] = bload_elem<double, 0>(rb, off_b + p * step);
 #pragma unroll
-        for (int p = 0; p < NP2; ++p) {
-            const int q = p * RPP2 + lr;
-#pragma unroll
-            for (int e = 0; e < VE; ++e) b[p].d[e] = b[p].d[e] + tile[lc + e][q];
-            if constexpr (VE == 2)
-                bstore16<AUX_ST>(rs[p], off, b[p].v);
-            else
-                bstore_elem<double, AUX_ST>(rs[p], off, b[p].d[0]);
-        }
-    }
+    for (int p = 0; p < NP; ++p) bstore_elem<double, 2>(rb, off_b + p * step, x[p] + tile[c][p * RPP + r]);
 }
 
 // One 128 x 128 tile of A on 1024 threads, in two halves through 66 KiB of
@@ -303,13 +347,31 @@ int transpose_args(int order, const double *A, const double *B)
 
 int g_tr_shape = -1, g_tr_mode = -1;  // -1: the defaults below
 
-template <int TR, int TC, int VE, int NTH = kTThreads>
-int launch_shape(TransposeArgs a, hipStream_t s)
+template <int TR, int TC, int NTH = 256>
+int launch_shape(TransposeArgs a, bool large, hipStream_t s)
 {
     a.ntr = (a.order + TR - 1) / TR;
     a.ntc = (a.order + TC - 1) / TC;
     const unsigned blocks = (unsigned)a.ntr * (unsigned)a.ntc;
-    hipLaunchKernelGGL((transpose_kernel<TR, TC, VE, 1, NTH>), dim3(blocks), dim3(NTH), 0, s, a);
+    // large: one workgroup per CU of the 64 x 128 tiles (more than half of
+    // its LDS each)
+    constexpr size_t lds = sizeof(double) * TR * (TC + 1), half = 80u * 1024u;
+    const size_t dyn = large && lds > half / 2 && lds < half ? half + 4096u - lds : 0;
+    if (a.order & 1)
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, false, true>), dim3(blocks), dim3(NTH), 0, s, a);
+    else if (large)
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, true, false>), dim3(blocks), dim3(NTH), dyn, s, a);
+    else
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, false, false>), dim3(blocks), dim3(NTH), 0, s, a);
+    return check_hip(hipGetLastError(), "transpose launch");
+}
+
+int launch_8b(TransposeArgs a, hipStream_t s)
+{
+    a.ntr = (a.order + 63) / 64;
+    a.ntc = a.ntr;
+    const unsigned blocks = (unsigned)a.ntr * (unsigned)a.ntc;
+    hipLaunchKernelGGL(transpose_kernel_8b, dim3(blocks), dim3(256), 0, s, a);
     return check_hip(hipGetLastError(), "transpose launch");
 }
 
@@ -322,23 +384,46 @@ int launch_2h(TransposeArgs a, hipStream_t s)
     return check_hip(hipGetLastError(), "transpose launch");
 }
 
+// The rule, with times on MI355X in us at each order:
+//  - Up to 1024, 32 x 64 tiles: enough workgroups for the chip (order 512:
+//    2.7, 64 x 128 tiles 4.2; 1000: 5.7 against 6.4; at 1400 they lose, 11.2
+//    against 9.4).
+//  - Up to 4096 64 x 128 tiles, loads and stores through the caches: both
+//    matrices stay in the 256 MB of the last one (order 2000: 19; 4096: 79,
+//    93 non-temporal; 64 x 64 tiles in 8-byte accesses at 3001: 56, these 48).
+//  - Above, rows on 64-byte boundaries: the same tiles, everything
+//    non-temporal and one workgroup at a time on a CU: order 32768 6005 (two
+//    workgroups 6150, only the stores non-temporal 6540), 16384 1490 (1520,
+//    1630), 9000 529 (533, 598), 20004 3071 (3106, 3379).
+//  - Rows off them share cache lines between tiles, and what one tile leaves
+//    of a line must wait in the cache for the next: 32 x 32 tiles without
+//    hints (order 10002 685, the tiles above 817 and with only the stores
+//    non-temporal 787; 16380 1744, 2098, 2043).  From 20004 on rows on
+//    32-byte boundaries do better with the tiles above (30004: 6975 against
+//    7837).
+//  - Odd orders and matrices off 16-byte boundaries: 64 x 64 tiles in 8-byte
+//    accesses (order 12289 1091, 32 x 32 tiles 1192, 64 x 128 1251).
 int launch_transpose(int order, double *A, double *B, hipStream_t s)
 {
     TransposeArgs a{A, B, order, 0, 0, g_tr_mode < 0 ? 0 : g_tr_mode};
-    const bool vec = order % 2 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
-    if (!vec) return launch_shape<kT, kT, 1>(a, s);
-    // default: 64 x 128 tiles in row-major order, measured best on MI355X at
-    // order 32768 (5.24 TB/s; 64 x 64: 4.95, every other shape/order <= 5.21)
-    switch (g_tr_shape < 0 ? 2 : g_tr_shape) {
-    case 1: return launch_shape<128, 64, 2>(a, s);
-    case 2: return launch_shape<64, 128, 2>(a, s);
-    case 3: return launch_shape<32, 64, 2>(a, s);
-    case 4: return launch_shape<128, 128, 2, 1024>(a, s);
-    case 5: return launch_shape<32, 256, 2>(a, s);
-    case 6: return launch_shape<256, 32, 2>(a, s);
-    case 7: return launch_shape<64, 128, 2, 512>(a, s);
-    case 8: return launch_2h(a, s);
-    default: return launch_shape<64, 64, 2>(a, s);
+    const bool aligned = order % 2 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
+    const bool large = order > 4096;
+    if (large && !aligned) return launch_8b(a, s);
+    if (large && g_tr_shape < 0 && (order % 4 != 0 || (order % 8 != 0 && order <= 16384)))
+        return launch_shape<32, 32>(a, false, s);
+    const int shape = order <= 1024 ? 3 : 2;
+    switch (g_tr_shape < 0 ? shape : g_tr_shape) {
+    case 1: return launch_shape<128, 64>(a, large, s);
+    case 2: return launch_shape<64, 128>(a, large, s);
+    case 3: return launch_shape<32, 64>(a, large, s);
+    case 4: return launch_shape<128, 128, 1024>(a, large, s);
+    case 5: return launch_shape<32, 256>(a, large, s);
+    case 6: return launch_shape<256, 32>(a, large, s);
+    case 7: return launch_shape<64, 128, 512>(a, large, s);
+    case 8:
+        if (aligned) return launch_2h(a, s);
+        return launch_shape<64, 64>(a, large, s);
+    default: return launch_shape<64, 64>(a, large, s);
     }
 }
 

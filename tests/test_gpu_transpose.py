@@ -100,3 +100,23 @@ def test_transpose_tile_shapes_do_not_change_results(gpu, oracle):
     finally:
         K.check(L.prk_set_transpose_variant(-1, -1))
     assert L.prk_set_transpose_variant(9, 0) == -1
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("order", [31, 33, 1023, 1024, 1025, 1026, 1151, 4095, 4096, 4097, 4098, 4100, 4104])
+def test_transpose_rule_edges(gpu, order, offset):
+    # both sides of every line of the tiling rule, odd and even, on 16-byte
+    # boundaries (offset 0) and off them: one rounding per element on both
+    # sides, so the bits of plain torch; nothing past the matrices is written
+    print(f"transpose order={order} offset={offset}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(order)
+    base = [torch.full((order * order + 4,), 7.0, dtype=torch.float64, device=gpu) for _ in range(2)]
+    A, B = (b[offset:offset + order * order].view(order, order) for b in base)
+    for m in (A, B):
+        m.copy_(torch.rand((order, order), generator=gen, device=gpu, dtype=torch.float64))
+    rB, rA = B + A.t(), A + 1.0
+    K.transpose(A, B)
+    assert torch.equal(A.view(torch.int64), rA.view(torch.int64))
+    assert torch.equal(B.view(torch.int64), rB.view(torch.int64))
+    for b in base:
+        assert bool((b[:offset] == 7.0).all() and (b[offset + order * order:] == 7.0).all())
