@@ -104,14 +104,14 @@ __device__ inline void init_tile(const BGrid &g, int c0, int r0, int r1, int lan
     constexpr int V = DTypeTraits<DT>::V, ES = (int)sizeof(T);
     const unsigned row_bytes = (unsigned)(g.pitch * ES);
     const int cm = c0 + lane * V;
-    for (int r = r0; r < r1; ++r) {
+    uint64_t state = seeded_state(g.seed, (uint64_t)r0 * (uint64_t)g.n + cm);
+    for (int r = r0; r < r1; ++r, state += (uint64_t)g.n * kSeedStep) {
         union { u32x4 v; T e[V]; } x, z;
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             const int c = cm + v;
             double val = 0.0;
-            if (c < g.n)
-                val = g.init_kind == 0 ? (double)(r + c) : seeded_value(g.seed, (uint64_t)r * (uint64_t)g.n + c);
+            if (c < g.n) val = g.init_kind == 0 ? (double)(r + c) : seeded_of_state(state + v * kSeedStep);
             if constexpr (DT == F64) {
                 x.e[v] = val;
                 z.e[v] = 0.0;

@@ -155,11 +155,16 @@ inline size_t dtype_size(int dt) { return dt == F64 ? 8 : dt == F32 ? 4 : 2; }
 
 // ---------------------------------------------------------------------------
 // Seeded initial values: SplitMix64 of (seed, idx), top 53 bits as a uniform
-// u in [0,1), value 2u-1 (exact in double).  Same on host and device.
+// u in [0,1), value 2u-1 (exact in double).  Same on host and device.  The
+// generator's state is seed + (idx + 1) * kSeedStep: neighbouring elements
+// add kSeedStep instead of multiplying.
 // ---------------------------------------------------------------------------
-__host__ __device__ inline double seeded_value(uint64_t seed, uint64_t idx)
+constexpr uint64_t kSeedStep = 0x9E3779B97F4A7C15ull;
+
+__host__ __device__ inline uint64_t seeded_state(uint64_t seed, uint64_t idx) { return seed + (idx + 1) * kSeedStep; }
+
+__host__ __device__ inline double seeded_of_state(uint64_t z)
 {
-    uint64_t z = seed + (idx + 1) * 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z = z ^ (z >> 31);
