@@ -294,6 +294,63 @@ __device__ inline void pair_sums_f64(const double *const (&rows)[2 * R + 1], dou
     if constexpr (C + 2 <= c_hi) pair_sums_f64<P, R, C + 2>(rows, s);
 }
 
+// The same for the two columns of two output rows (grid stencils from
+// R = kGridPairRadius): chain (m, ch) is output row o + m, column ch, and
+// rows[k] holds input row o - R + k, k = 0 .. 2R+1.  The four chains advance
+// together, element by element down each column.  A row read from LDS serves
+// both output rows (2R + 2 reads per column pair instead of two times
+// 2R + 1), and a product of one element and one ring's weight serves every
+// chain that has it: subtracting x * |w| is adding x * -|w|, so taps of
+// either sign share it (110 products per point at R = 5 become about 60).
+template <int R, int M, int CH, int COL, int K>
+__device__ inline void pair2_tap_f64(double x, double &s)
+{
+#pragma clang fp contract(off)
+    constexpr int dj = COL - CH, di = K - M - R;
+    if constexpr (dj >= -R && dj <= R && di >= -R && di <= R) {
+        constexpr double w = weight_ab(GRID, R, dj, di);
+        if constexpr (w != 0.0) {
+            const double p = x * (w < 0.0 ? -w : w);
+            if constexpr (dj == -R && di == -R)  // the chain's first tap
+                s = w < 0.0 ? -p : p;
+            else
+                s = w < 0.0 ? s - p : s + p;
+        }
+    }
+}
+
+template <int R, int COL, int K>
+__device__ inline void pair2_column_f64(const double (&x)[2 * R + 2], double (&s)[2][2])
+{
+    pair2_tap_f64<R, 0, 1, COL, K>(x[K], s[0][1]);
+    pair2_tap_f64<R, 1, 1, COL, K>(x[K], s[1][1]);
+    pair2_tap_f64<R, 0, 0, COL, K>(x[K], s[0][0]);
+    pair2_tap_f64<R, 1, 0, COL, K>(x[K], s[1][0]);
+    if constexpr (K < 2 * R + 1) pair2_column_f64<R, COL, K + 1>(x, s);
+}
+
+template <int R, int C>
+__device__ inline void pair2_sums_f64(const double *const (&rows)[2 * R + 2], double (&s)[2][2])
+{
+    constexpr int c_hi = (R & 1) ? R + 1 : R;
+    double x[2][2 * R + 2];
+#pragma unroll
+    for (int k = 0; k < 2 * R + 2; ++k) {
+        union { u32x4 v; double e[2]; } u;
+        u.v = *(const u32x4 *)(rows[k] + C);
+        x[0][k] = u.e[0];
+        x[1][k] = u.e[1];
+    }
+    pair2_column_f64<R, C, 0>(x[0], s);
+    pair2_column_f64<R, C + 1, 0>(x[1], s);
+    // The four chains end here: left to itself the compiler forms row o + 1's
+    // later, where it is stored, and keeps every element until then (over 400
+    // registers at R = 5 instead of 161).  The fence as in pair_sums_f64.
+    __asm__ volatile("" : "+v"(s[0][0]), "+v"(s[0][1]), "+v"(s[1][0]), "+v"(s[1][1]));
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (C + 2 <= c_hi) pair2_sums_f64<R, C + 2>(rows, s);
+}
+
 // Reduced-precision forms.  The window of a row is the columns [-HP, V+HP)
 // around the lane's own V columns (window index i = column i - HP); a row
 // whose taps reach MAXD columns to either side needs the indices
@@ -527,9 +584,22 @@ __device__ inline void compute_points(const typename DTypeTraits<DT>::T *const (
 template <int DT, int P, int R>
 constexpr bool star_reg_ring() { return P == STAR && R >= (DT == F32 ? 4 : 6); }
 
+// The FP64 grid sweeps that take two output rows at a time
+// (wave_tile_grid2).  They are bound by their VALU issue and LDS reads.
+// Measured on MI355X at n = 16384, one row at a time -> two, the same tiling:
+// R=3 1706 -> 1577 us, R=4 2057 -> 1806, R=5 2793 -> 2322, R=6 3473 -> 2858,
+// R=7 4560 -> 3647.  At R = 8 the 18-row ring would leave one workgroup per
+// CU (83 KB); below R = 3 the sweep is at HBM's rate.
+constexpr int kGridPairRadius = 3;
+template <int DT, int P, int R>
+constexpr bool grid_row_pairs() { return DT == F64 && P == GRID && R >= kGridPairRadius && R <= 7; }
+
 // LDS ring rows per wave of the sweep kernel, and its static LDS per workgroup.
 template <int DT, int P, int R>
-constexpr int sweep_ring_rows() { return star_reg_ring<DT, P, R>() ? R + 1 : 2 * R + 1; }
+constexpr int sweep_ring_rows()
+{
+    return star_reg_ring<DT, P, R>() ? R + 1 : grid_row_pairs<DT, P, R>() ? 2 * R + 2 : 2 * R + 1;
+}
 
 template <int DT, int P, int R>
 constexpr size_t sweep_lds_bytes()
@@ -1138,6 +1208,139 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
 }
 
 
+// wave_tile for the FP64 grid stencils from R = kGridPairRadius: the same
+// loads, stores and sums, two rows at a time.  The LDS ring holds 2R + 2
+// rows; step s parks rows lo + 2s and lo + 2s + 1 and computes the two output
+// rows R above them.  PF pairs of rows are in flight.
+template <int R, bool FUSE, int MODE, int PF, int NT>
+__device__ inline void wave_tile_grid2(const void *in_, void *in_next_, void *out_, long long pitch, int n,
+                                       const RowSpan &sp, int c0, int r0, int r1, int pad_writable,
+                                       double *ring_base, int lane, u32x4 *stash_lds)
+{
+#pragma clang fp contract(off)
+    // wave-uniform: only the first and last strips of a row hold frame columns
+    const bool edge = c0 < R || c0 + SweepGeom<F64, R>::SW > n - R;
+    typedef SweepGeom<F64, R> G;
+    typedef double T;
+    constexpr int DT = F64, V = G::V, HP = G::HP, NH = G::NH, LR = G::LR;
+    constexpr int S = 2 * R + 2;  // LDS ring rows
+    constexpr int ES = (int)sizeof(T);
+    constexpr int AUX_STREAM = (NT & 1) ? 2 : 0;
+
+    const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
+    const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
+    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
+
+    const T *in = (const T *)in_;
+    T *in_next = (T *)in_next_;
+    T *out = (T *)out_;
+    const unsigned ld_bytes = (unsigned)(pitch * ES);
+    const unsigned st_bytes = pad_writable ? ld_bytes : (unsigned)(n * ES);
+    // wave-uniform: the strip holds a vector with columns on both sides of n
+    const bool ragged = !pad_writable && n % V != 0 && c0 + G::SW > n;
+
+    const int cm = c0 + lane * V;
+    const int ch = lane < NH ? c0 - HP + lane * V : c0 + G::SW + (lane - NH) * V;
+    const int lh = lane < NH ? lane * V : HP + G::SW + (lane - NH) * V;
+    const unsigned off_main = (unsigned)(cm * ES);
+    const unsigned off_halo = lane < 2 * NH ? (unsigned)(ch * ES) : kOOB;
+
+    T(*ring)[LR] = (T(*)[LR])ring_base;
+
+    RowRegs<T, V> buf[PF][2];
+    auto issue = [&](RowRegs<T, V> &r, int ri) {
+        const bool row_ok = ri < hi;
+        const int rr = row_ok ? ri : lo;
+        const bool end = rr + 1 == sp.nrows;
+        const __amdgpu_buffer_rsrc_t rin = row_rsrc(in + (long long)rr * pitch, row_load_bytes<MODE>(ld_bytes, end));
+        const int o = ri - R;
+        const bool out_ok = o >= olo && o < ohi;
+        // rows of out that are read are interior: never the last
+        const __amdgpu_buffer_rsrc_t rout =
+            row_rsrc(out + (long long)(out_ok ? o : olo) * pitch, row_load_bytes<MODE>(ld_bytes, !out_ok));
+        r.main.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_main : kOOB, end);
+        r.halo.v = load_row_vec<T, V, MODE, 0>(rin, row_ok ? off_halo : kOOB, end);
+        r.outv.v = load_row_vec<T, V, MODE, AUX_STREAM>(rout, out_ok ? off_main : kOOB, false);
+    };
+
+#pragma unroll
+    for (int k = 0; k < PF; ++k)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) issue(buf[k][m], lo + 2 * k + m);
+
+    int slot = 0;  // ring slot of row ri: (ri - lo) % S, even
+    for (int base = lo; base < hi; base += 2 * PF) {
+#pragma unroll
+        for (int k = 0; k < PF; ++k) {
+            const int ri = base + 2 * k;
+            RowRegs<T, V> cur[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                cur[m] = buf[k][m];
+                issue(buf[k][m], ri + 2 * PF + m);
+            }
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                *(u32x4 *)&ring[slot + m][HP + lane * V] = cur[m].main.v;
+                if (lane < 2 * NH) *(u32x4 *)&ring[slot + m][lh] = cur[m].halo.v;
+                if constexpr (FUSE) {
+                    const bool nx_ok = ri + m >= ulo && ri + m < uhi;
+                    const __amdgpu_buffer_rsrc_t rnx =
+                        row_rsrc(in_next + (long long)(nx_ok ? ri + m : r0) * pitch, st_bytes);
+                    union { u32x4 v; T e[V]; } nx;
+                    plus_one<DT, V>(cur[m].main.e, nx.e);
+                    store_next_vec<T, V, MODE, AUX_STREAM>(rnx, nx_ok ? off_main : kOOB, cm, n, ragged, nx.v);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+            // Output rows o and o + 1: rows o - R .. o + 1 + R are the whole
+            // ring, the oldest in slot + 2.  Before the first output row the
+            // ring is still filling; past the last one o + 1 may be no output
+            // row (its sum is formed from what the ring holds and dropped).
+            const int o = ri - R;
+            if (o >= olo && o < ohi) {
+                const T *rows[S];
+#pragma unroll
+                for (int j = 0; j < S; ++j) {
+                    int s2 = slot + 2 + j;
+                    s2 = s2 >= S ? s2 - S : s2;
+                    rows[j] = &ring[s2][HP + lane * V];
+                }
+                double sum[2][V];
+                pair2_sums_f64<R, (R & 1) ? -R - 1 : -R>(rows, sum);
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    if (o + m >= ohi) break;  // uniform
+                    union { u32x4 v; T e[V]; } res;
+#pragma unroll
+                    for (int v = 0; v < V; ++v) res.e[v] = cur[m].outv.e[v] + sum[m][v];
+                    const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)(o + m) * pitch, st_bytes);
+                    if constexpr (MODE != MODE_ELEM) {
+                        if (!edge) {
+                            bstore16<AUX_STREAM>(rout, off_main, res.v);
+                        } else {
+                            edge_store<T, V, ES, AUX_STREAM>(rout, off_main, res.v, c0, n, R, stash, o + m - olo);
+                            if (stash && o + m + 1 == ohi)
+                                flush_edge_stash<T, V, ES, AUX_STREAM>(stash, out, pitch, n, R, c0, G::SW, olo,
+                                                                       ohi - olo);
+                        }
+                    } else {
+                        unsigned off[V];
+                        out_offsets<V, ES>(c0, n, R, off);
+#pragma unroll
+                        for (int v = 0; v < V; ++v) bstore_elem<T, AUX_STREAM>(rout, off[v], res.e[v]);
+                    }
+                }
+            }
+            slot = slot + 2 == S ? 0 : slot + 2;
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Reduced-precision sweeps at small R from a register ring of widened row
 // windows.  The LDS-ring sweep widens every value it reads, so each input
@@ -1418,6 +1621,10 @@ void sweep_kernel(SweepArgs a)
         wave_tile_star<DT, R, FUSE, MODE, PF, NT>(a.in, a.in_next, a.out, a.pitch, a.n, a.span, strip * G::SW, r0,
                                                   r1, a.pad_writable, &lds[wave][0][0], lane,
                                                   a.stash ? sweep_dyn_lds : nullptr);
+    else if constexpr (grid_row_pairs<DT, P, R>())
+        wave_tile_grid2<R, FUSE, MODE, PF, NT>(a.in, a.in_next, a.out, a.pitch, a.n, a.span, strip * G::SW, r0, r1,
+                                               a.pad_writable, &lds[wave][0][0], lane,
+                                               a.stash ? sweep_dyn_lds : nullptr);
     else
         wave_tile<DT, P, R, FUSE, MODE, PF, NT, 0>(a.in, a.in_next, a.out, a.pitch, a.n, a.span, strip * G::SW,
                                                    r0, r1, a.pad_writable, &lds[wave][0][0], lane,

@@ -484,3 +484,24 @@ def test_ragged_and_misaligned_rows_bitwise(gpu, oracle, pattern, radius, dtype,
             assert np.array_equal(g, ref.view(g.dtype)), (n, pitch)
         for b in base:
             assert bool((b[:, n:] == 3.0).all()), (n, pitch)
+
+
+@pytest.mark.parametrize("radius", [3, 4, 5, 6, 7, 8])
+def test_grid_row_pairs_bitwise(gpu, oracle, radius):
+    # the FP64 grid sweeps take output rows in pairs: row blocks of odd and
+    # even heights down to one row, blocks that end on the first row of a
+    # pair, and more rows than the edge stash holds
+    L = K.lib()
+    try:
+        for n in (2 * radius + 1, 2 * radius + 2, 129, 140):
+            ref_out, ref_in = oracle.run(K.GRID, radius, n, 32, 1, 1, n)
+            for rows in (1, 2, 3, 8, 13, 64, 65, 128):
+                print(f"grid R={radius} n={n} rows={rows}", flush=True)
+                K.check(L.prk_set_rows_per_wave(rows))
+                b0, b1, out = (K.alloc_grid(n, K.F64) for _ in range(3))
+                K.init(K.INIT_SEEDED, n, K.F64, b0, out)
+                fb, _ = K.run(K.GRID, radius, K.F64, 1, b0, b1, out)
+                assert np.array_equal(out.contiguous().cpu().numpy().view(np.uint64), ref_out.view(np.uint64))
+                assert np.array_equal((b0, b1)[fb].contiguous().cpu().numpy().view(np.uint64), ref_in.view(np.uint64))
+    finally:
+        K.check(L.prk_set_rows_per_wave(0))
