@@ -37,18 +37,63 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 
 }  // namespace
 
-// Measured defaults on MI355X (n = 16384 and 30000): a 3-row non-temporal
-// pipeline, two workgroups per CU (four for BF16, whose eight columns per
-// lane make each row step longer), row blocks growing with the radius so
-// the 2R halo rows each block re-reads stay a small fraction.
+// Measured defaults on MI355X: a 3-row non-temporal pipeline, and by size:
+//  - Large grids take the row blocks and workgroups per CU that were fastest
+//    at n = 16384 for each stencil: the HBM-bound sweeps want two workgroups
+//    per CU, those with longer row steps as many as fit.  Against the rule
+//    below for the middle: FP64 star R=8 1683 -> 1547 us; FP32 star R=5 797
+//    -> 730, grid R=5 1010 -> 901; BF16 star R=1 404 -> 380, grid R=6 942 ->
+//    853.  The FP64 grids from R = 3 and the FP32 grid R=5, which are bound
+//    by their arithmetic, take theirs at every size (FP64 grid R=5, n = 5000:
+//    272 -> 213).
+//  - In the middle one height per radius, growing so that the 2R halo rows
+//    each block re-reads stay a small share, and two workgroups per CU (four
+//    in BF16): what was fastest at 16384 loses up to 15 % between 2000 and
+//    8000, where the turns of the chip count (FP64 star R=5, n = 6000: 203
+//    us, 8 rows 220).
+//  - A grid of less than three (BF16: two) turns of two workgroups per CU takes the
+//    height that fills its turns best, the last one of which may be nearly
+//    empty, against the share of halo rows (FP64 star R=4, n = 2000: 16 rows
+//    are 0.98 of a turn, 25 us; 12 rows 1.3 turns, 32 us; FP64 grid R=5, n =
+//    1000: 8 rows 16 us, 24 rows 44).  Stars and grids of R <= 2 keep 8 rows.
 prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
 {
-    (void)pattern;
+    static const signed char kRows[3][2][kMaxRadius] = {
+        {{8, 8, 12, 12, 8, 8, 12, 24}, {8, 8, 12, 24, 32, 48, 48, 32}},
+        {{8, 8, 12, 12, 12, 12, 16, 16}, {8, 8, 12, 16, 32, 48, 48, 48}},
+        {{8, 8, 12, 12, 12, 12, 24, 24}, {12, 12, 12, 32, 32, 32, 32, 32}}};
+    static const signed char kWgs[3][2][kMaxRadius] = {
+        {{2, 2, 2, 2, 4, 4, 4, 4}, {2, 2, 4, 4, 4, 4, 4, 4}},
+        {{2, 2, 2, 2, 2, 2, 2, 2}, {2, 2, 2, 2, 4, 4, 4, 4}},
+        {{2, 2, 2, 4, 4, 4, 4, 4}, {2, 3, 4, 4, 4, 4, 4, 4}}};
+    const int d = dtype == F32 || dtype == BF16 ? dtype : F64, p = pattern == GRID ? 1 : 0;
+    const int R = std::max(1, std::min(radius, kMaxRadius));
     prk_tuning t;
     t.variant = 5;
     t.order = 1;
-    t.wgs_per_cu = dtype == BF16 ? 4 : 2;
-    int rows = dtype == BF16 ? 12 : (radius <= 2 ? 8 : radius == 3 ? 12 : radius == 4 ? 16 : 24);
+    int rows = d == BF16 ? 12 : R <= 2 ? 8 : R == 3 ? 12 : R == 4 ? 16 : 24;
+    t.wgs_per_cu = d == BF16 ? 4 : 2;
+    const bool large = n >= (d == F64 ? 8000 : 12000);
+    if (large || (p == 1 && ((d == F64 && R >= 3) || (d == F32 && R == 5)))) {
+        rows = kRows[d][p][R - 1];
+        t.wgs_per_cu = kWgs[d][p][R - 1];
+    }
+    const int lanes = d == F64 ? 128 : d == F32 ? 256 : 512;  // columns of a strip
+    const long long groups = ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock, turn = 512;
+    auto tiles = [&](int h) { return groups * ((n + h - 1) / h); };
+    if ((R >= 3 || d == BF16) && tiles(rows) < (d == BF16 ? 2 : 3) * turn) {
+        static const int kHeights[] = {8, 12, 16, 24, 32};
+        double best = 0.0;
+        for (int h : kHeights) {
+            if (d == BF16 && h > 16) break;  // its row steps are long: 24 and 32 rows lose however they fill
+            const long long turns = (tiles(h) + turn - 1) / turn;
+            const double score = (double)tiles(h) / (double)(turns * turn) * h / (h + 0.6 * R);
+            if (score > best) {
+                best = score;
+                rows = h;
+            }
+        }
+    }
     t.rows_per_wave = std::max(1, std::min(rows, n));
     t.gbs = 0.0;
     return t;
