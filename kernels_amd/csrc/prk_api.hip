@@ -754,6 +754,36 @@ int prk_l1norm_noalloc(int dtype, int n, long long pitch, int radius, const void
     return enqueue_l1norm(dtype, n, pitch, radius, out, d_norm, (DD *)ptr, (hipStream_t)stream);
 }
 
+// The two events of a thread's prk_run calls, made once per thread and device
+// and given back when the thread ends.  prk_run returns only once its last
+// event has passed, so a call finds them idle.
+struct RunEvents {
+    int device = -1;
+    hipEvent_t e[2] = {nullptr, nullptr};
+    void release()
+    {
+        for (hipEvent_t &x : e) {
+            if (x) (void)hipEventDestroy(x);
+            x = nullptr;
+        }
+        device = -1;
+    }
+    ~RunEvents() { release(); }
+    int get()
+    {
+        int dev = 0;
+        int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
+        if (rc || dev == device) return rc;
+        release();
+        for (hipEvent_t &x : e)
+            if (!rc) rc = check_hip(hipEventCreate(&x), "event create");
+        if (rc) release();
+        else device = dev;
+        return rc;
+    }
+};
+static thread_local RunEvents t_run_events;
+
 int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iterations, void *buf0, void *buf1,
             void *out, void *stream, int *final_in_buf, double *avg_seconds)
 {
@@ -763,12 +793,8 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     int rc = plan_sweep(pattern, radius, dtype, n, pitch, buf0, buf1, out, 0, &p);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    hipEvent_t e0, e1;
-    if ((rc = check_hip(hipEventCreate(&e0), "event create"))) return rc;
-    if ((rc = check_hip(hipEventCreate(&e1), "event create"))) {
-        (void)hipEventDestroy(e0);
-        return rc;
-    }
+    if ((rc = t_run_events.get())) return rc;
+    const hipEvent_t e0 = t_run_events.e[0], e1 = t_run_events.e[1];
     // Sweep 0 runs by itself; the timed sweeps run in `passes` passes over the
     // grid (pass.hpp) of nearly equal length.  The final in must end in the
     // buffer that one sweep per pass would leave it in, so the number of
@@ -796,9 +822,10 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     if (rc == PRK_OK) rc = check_hip(hipEventSynchronize(e1), "event sync");
     float ms = 0.0f;
     if (rc == PRK_OK) rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "event elapsed");
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (rc) return rc;
+    if (rc) {
+        t_run_events.release();  // a failed run may leave them recorded
+        return rc;
+    }
     if (final_in_buf) *final_in_buf = cur;
     if (avg_seconds) *avg_seconds = 1e-3 * (double)ms / iterations;
     return PRK_OK;
