@@ -21,6 +21,8 @@
 // R=2 1410 -> 112 us, star R=5 1532 -> 362, grid R=2 1408 -> 249, grid R=3
 // 1705 -> 615; FP32 star R=2 715 -> 55, grid R=3 739 -> 170, grid R=5 1014
 // -> 397; BF16 star R=2 403 -> 102, star R=8 494 -> 396, grid R=2 406 -> 204.
+// Two vectors per lane (fewer halo columns to refresh) gave the FP64 star R=3
+// 5 % over 50 sweeps and cost every pass twice its loading and storing time.
 //
 // Mapping.  A lane owns V columns (16 bytes) of M output rows and keeps
 // their window in registers: (M+2R) x (V+2R) values, for the stars without
@@ -50,6 +52,18 @@ constexpr int pass_rows()
 
 template <int DT, int P, int R>
 constexpr bool pass_ok() { return pass_rows<DT, P, R>() > 0; }
+
+// Sweeps from which a pass beats that many sweeps on their own: loading a
+// wide window takes longer than the two sweeps save (n = 16384, two sweeps:
+// FP32 grid R=5 1074 us each in a pass, 870 alone; BF16 star R=7 485, 450;
+// with three 746 and 409).
+constexpr int pass_min_sweeps(int pattern, int radius, int dtype)
+{
+    return (pattern == GRID && ((dtype == F64 && radius >= 3) || (dtype == F32 && radius >= 5))) ||
+                   (dtype == BF16 && radius >= 7)
+               ? 3
+               : 2;
+}
 
 template <int DT, int... I>
 constexpr bool pass_built_dtype(int pattern, int radius, std::integer_sequence<int, I...>)
@@ -352,7 +366,7 @@ struct PassArgs {
 // A workgroup is four waves on row blocks below one another of one strip of
 // 64*V columns; workgroups run along the strips of a row band first.
 template <int DT, int P, int R, bool ALIGNED>
-__global__ __launch_bounds__(kThreads) void pass_kernel(PassArgs a)
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void pass_kernel(PassArgs a)
 {
     constexpr int V = DTypeTraits<DT>::V;
     const int band = blockIdx.x / a.nstrips, strip = blockIdx.x - band * a.nstrips;

@@ -805,6 +805,7 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     if (!overridden && pass_built(pattern, radius, dtype) && (p.mode != MODE_ELEM || dtype == BF16)) {
         passes = (iterations + kMaxPassSweeps - 1) / kMaxPassSweeps;
         passes += (passes ^ iterations) & 1;
+        if (iterations / passes < pass_min_sweeps(pattern, radius, dtype)) passes = iterations;
     }
     void *bufs[2] = {buf0, buf1};
     int cur = 0;
