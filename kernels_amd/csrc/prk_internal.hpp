@@ -64,7 +64,8 @@ int launch_sweep_f32(const SweepPlan &p, const void *in, void *in_next, void *ou
 int launch_sweep_bf16(const SweepPlan &p, const void *in, void *in_next, void *out, hipStream_t s);
 
 // Enqueue one pass of `sweeps` sweeps over a whole grid (pass.hpp): in_next
-// gets in after that many refreshes.  Only where pass_built.
+// gets in after that many refreshes.  Only where pass_built.  With sweeps == 0
+// the kernel's code is loaded and nothing launched.
 int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
 int launch_pass_f64(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
 int launch_pass_f32(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
@@ -74,6 +75,5 @@ int launch_pass_bf16(const SweepPlan &p, int sweeps, const void *in, void *in_ne
 // interrupted one bounded (star R=2 FP64 at n = 30000: 256 sweeps take about
 // 0.1 s).
 constexpr int kMaxPassSweeps = 256;
-
 
 }  // namespace prk

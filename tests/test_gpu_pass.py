@@ -85,3 +85,20 @@ def test_passes_equal_single_sweeps(gpu):
         finally:
             K.check(K.lib().prk_set_rows_per_wave(0))
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+def test_first_run_is_timed_without_loading_code(gpu):
+    """The time a fresh process reports for its first run is that of the
+    sweeps.  Loading the pass kernel's code takes about 0.6 ms, 60 us for each
+    of 10 sweeps, where a sweep by itself takes 9; the least of five processes
+    is under 30."""
+    import re
+    import subprocess
+    from pathlib import Path
+
+    exe = Path(K.__file__).parent / "prk-stencil"
+    times = []
+    for _ in range(5):
+        text = subprocess.run([str(exe), "10", "1000"], capture_output=True, text=True, timeout=60, check=True).stdout
+        times.append(float(re.search(r"Avg time \(s\):\s*(\S+)", text).group(1)))
+    assert min(times) < 30e-6, times
