@@ -194,7 +194,7 @@ __device__ inline void pass_stage(const BGrid &g, int k, int tile, int lane)
     NormSum ns;
     pass_tile<DT, P, R, true>((p & 1) ? g.buf1 : g.buf0, (p & 1) ? g.buf0 : g.buf1, g.out, g.pitch, g.n,
                               (strip * 64 + lane) * V, r0, min(r0 + g.pass_rows, g.n), sweeps, (int)g.pitch, k == 0,
-                              last, ns);
+                              last, false, ns);
     if (last) {
         const DDv part = wave_reduce_dd(DDv{ns.sum, ns.comp});
         if (lane == 0) g.partials[tile] = part;

@@ -92,11 +92,11 @@ constexpr bool power_of_two(double w)
 
 // Tap K of one FP64 sum, in the generator's order.  A product by a power of
 // two is exact unless it falls below the normal range, so there the multiply
-// and the add are one fma with the same result.  No product falls that low:
-// a value the library refreshed (in + 1) or seeded itself is 0 or at least
-// 2^-53 in magnitude, and passes run on such values only (prk_run's first
-// sweep, which reads the caller's values, is a sweep of its own).
-template <int P, int R, int M, int V, int K>
+// and the add are one fma with the same result (FMA).  No product falls that
+// low for a value the library refreshed (in + 1) or seeded itself, which is 0
+// or at least 2^-53 in magnitude; the first sweep over a caller's values
+// multiplies and adds.
+template <int P, int R, int M, int V, bool FMA, int K>
 __device__ inline void pass_tap_f64(const double (&w)[M + 2 * R][V + 2 * R], double (&s)[M][V])
 {
 #pragma clang fp contract(off)
@@ -108,18 +108,18 @@ __device__ inline void pass_tap_f64(const double (&w)[M + 2 * R][V + 2 * R], dou
             const double x = w[m + R + t.di][v + R + t.dj];
             if constexpr (K == 0)
                 s[m][v] = x * t.w;
-            else if constexpr (power_of_two(t.w))
+            else if constexpr (FMA && power_of_two(t.w))
                 s[m][v] = __builtin_fma(x, t.w, s[m][v]);
             else
                 s[m][v] = s[m][v] + x * t.w;
         }
 }
 
-template <int P, int R, int M, int V, size_t... I>
+template <int P, int R, int M, int V, bool FMA, size_t... I>
 __device__ inline void pass_taps_f64(const double (&w)[M + 2 * R][V + 2 * R], double (&s)[M][V],
                                      std::index_sequence<I...>)
 {
-    (pass_tap_f64<P, R, M, V, (int)I>(w, s), ...);
+    (pass_tap_f64<P, R, M, V, FMA, (int)I>(w, s), ...);
 }
 
 // The reduced-precision sums of one output row: the pairs of the stars, the
@@ -224,10 +224,11 @@ struct NormSum {
 // n x n grid: in is read, in_next gets in after `sweeps` refreshes (columns
 // below st_cols), out is updated on the interior.  `first`: out holds
 // nothing yet and starts from zeros, frame included (columns below st_cols).
-// `last`: adds |out| over the lane's interior points to `norm`.
+// `last`: adds |out| over the lane's interior points to `norm`.  `any`: in
+// may hold any values (otherwise refreshed or seeded ones, pass_tap_f64).
 template <int DT, int P, int R, bool ALIGNED>
 __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, long long pitch, int n, int cm, int r0,
-                                 int r1, int sweeps, int st_cols, bool first, bool last, NormSum &norm)
+                                 int r1, int sweeps, int st_cols, bool first, bool last, bool any, NormSum &norm)
 {
 #pragma clang fp contract(off)
     typedef typename DTypeTraits<DT>::T T;
@@ -279,7 +280,9 @@ __device__ inline void pass_tile(const void *in_, void *in_next_, void *out_, lo
         for (int t = 0; t < sweeps; ++t) {
             C s[M][V];
             if constexpr (DT == F64) {
-                pass_taps_f64<P, R, M, V>(w, s, std::make_index_sequence<Stencil<P, R>::taps.count>{});
+                typedef std::make_index_sequence<Stencil<P, R>::taps.count> Taps;
+                if (any && t == 0) pass_taps_f64<P, R, M, V, false>(w, s, Taps{});
+                else pass_taps_f64<P, R, M, V, true>(w, s, Taps{});
             } else if constexpr (P == STAR) {
                 pass_pairs<R, M, V>(w, s, std::make_index_sequence<Stencil<P, R>::pairs.count>{});
             } else {
@@ -361,6 +364,7 @@ struct PassArgs {
     int nstrips;  // ceil(n / 64V)
     int rows;     // rows per wave, a multiple of M
     int sweeps;
+    int any;      // in may hold any values
 };
 
 // A workgroup is four waves on row blocks below one another of one strip of
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     if (r0 >= a.n) return;
     NormSum unused;
     pass_tile<DT, P, R, ALIGNED>(a.in, a.in_next, a.out, a.pitch, a.n, (strip * 64 + lane) * V, r0,
-                                 min(r0 + a.rows, a.n), a.sweeps, a.n, false, false, unused);
+                                 min(r0 + a.rows, a.n), a.sweeps, a.n, false, false, a.any, unused);
 }
 
 }  // namespace prk

@@ -2,8 +2,8 @@
 #include "sweep_launch.hpp"
 
 namespace prk {
-int launch_pass_f64(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
+int launch_pass_f64(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s)
 {
-    return launch_pass_dtype<F64>(p, sweeps, in, in_next, out, s);
+    return launch_pass_dtype<F64>(p, sweeps, any, in, in_next, out, s);
 }
 }  // namespace prk

@@ -105,12 +105,12 @@ int launch_sweep(const SweepPlan &p, const void *in, void *in_next, void *out, h
     return set_error(PRK_EINVAL, "unknown dtype %d", p.dtype);
 }
 
-int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
+int launch_pass(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s)
 {
     switch (p.dtype) {
-    case F64: return launch_pass_f64(p, sweeps, in, in_next, out, s);
-    case F32: return launch_pass_f32(p, sweeps, in, in_next, out, s);
-    case BF16: return launch_pass_bf16(p, sweeps, in, in_next, out, s);
+    case F64: return launch_pass_f64(p, sweeps, any, in, in_next, out, s);
+    case F32: return launch_pass_f32(p, sweeps, any, in, in_next, out, s);
+    case BF16: return launch_pass_bf16(p, sweeps, any, in, in_next, out, s);
     }
     return set_error(PRK_EINVAL, "unknown dtype %d", p.dtype);
 }
@@ -795,34 +795,50 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     hipStream_t s = (hipStream_t)stream;
     if ((rc = t_run_events.get())) return rc;
     const hipEvent_t e0 = t_run_events.e[0], e1 = t_run_events.e[1];
-    // Sweep 0 runs by itself; the timed sweeps run in `passes` passes over the
-    // grid (pass.hpp) of nearly equal length.  The final in must end in the
-    // buffer that one sweep per pass would leave it in, so the number of
-    // passes is odd or even as the number of sweeps is.  A tiling override
+    // The sweeps run in `passes` passes over the grid (pass.hpp) of nearly
+    // equal length.  The final in must end in the buffer that one sweep per
+    // pass would leave it in, so the number of passes is odd or even as the
+    // number of sweeps is.  Sweep 0 runs alone, untimed, unless it fits the
+    // passes of the others and saves one: an even number of iterations takes
+    // two passes, with sweep 0 one.  Measured with sweep 0 apart -> in the
+    // pass: star R=2 FP64 with init and norm, n = 30000, 100 iterations 42.1
+    // -> 37.9 ms, n = 1000, 10 iterations 81 -> 54 us; n = 16384, 2 / 50
+    // iterations, star R=1 FP32 2.91x / 1.45x, star R=8 BF16 1.19x / 1.01x,
+    // grid R=4 FP64 (the widest window) 1.14x / 1.01x.  A tiling override
     // asks for the sweep kernel itself: one sweep per pass then.
     const bool overridden = g_rows_per_wave > 0 || g_variant_override >= 0 || g_order >= 0 || g_wgs_per_cu >= 0;
-    int passes = iterations;
+    int alone = 1, passes = iterations;
     if (!overridden && pass_built(pattern, radius, dtype) && (p.mode != MODE_ELEM || dtype == BF16)) {
-        passes = (iterations + kMaxPassSweeps - 1) / kMaxPassSweeps;
-        passes += (passes ^ iterations) & 1;
-        if (iterations / passes < pass_min_sweeps(pattern, radius, dtype)) passes = iterations;
+        const auto fit = [](long long sweeps) {
+            const int k = (int)((sweeps + kMaxPassSweeps - 1) / kMaxPassSweeps);
+            return k + (int)((k ^ sweeps) & 1);
+        };
+        const long long all = (long long)iterations + 1;
+        const int joined = fit(all), apart = fit(iterations), least = pass_min_sweeps(pattern, radius, dtype);
+        if (joined < apart && all / joined >= least) {
+            alone = 0;
+            passes = joined;
+        } else if (iterations / apart >= least) {
+            passes = apart;
+        }
     }
+    const long long timed = (long long)iterations + 1 - alone;
     void *bufs[2] = {buf0, buf1};
     int cur = 0;
-    for (int it = 0, done = 0; it <= passes && rc == PRK_OK; ++it) {
-        if (it == 1) {
-            // While sweep 0 runs: a process's first pass would otherwise load
-            // its code between the events (0.6 ms, measured on a first run of
-            // n = 1000 whose passes take 20 us).
-            if (passes < iterations) rc = launch_pass(p, 0, buf0, buf1, out, s);
-            if (rc == PRK_OK) rc = check_hip(hipEventRecord(e0, s), "event record");
-        }
-        // sweeps left, spread over the passes left
-        const int sweeps = it == 0 ? 1 : (iterations - done) / (passes - it + 1);
-        if (rc == PRK_OK)
-            rc = sweeps == 1 ? launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s)
-                             : launch_pass(p, sweeps, bufs[cur], bufs[cur ^ 1], out, s);
-        if (it > 0) done += sweeps;
+    if (alone) {
+        rc = launch_sweep(p, buf0, buf1, out, s);
+        cur = 1;
+    }
+    // A process's first pass would otherwise load its code between the events
+    // (0.6 ms, measured on a first run of n = 1000 whose passes take 20 us).
+    if (rc == PRK_OK && passes < timed) rc = launch_pass(p, 0, false, buf0, buf1, out, s);
+    if (rc == PRK_OK) rc = check_hip(hipEventRecord(e0, s), "event record");
+    long long left = timed;
+    for (int it = 0; it < passes && rc == PRK_OK; ++it) {
+        const int sweeps = (int)(left / (passes - it));  // spread over the passes left
+        rc = sweeps == 1 ? launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s)
+                         : launch_pass(p, sweeps, !alone && it == 0, bufs[cur], bufs[cur ^ 1], out, s);
+        left -= sweeps;
         cur ^= 1;
     }
     if (rc == PRK_OK) rc = check_hip(hipEventRecord(e1, s), "event record");
@@ -834,7 +850,7 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
         return rc;
     }
     if (final_in_buf) *final_in_buf = cur;
-    if (avg_seconds) *avg_seconds = 1e-3 * (double)ms / iterations;
+    if (avg_seconds) *avg_seconds = 1e-3 * (double)ms / (double)timed;
     return PRK_OK;
 }
 

@@ -66,10 +66,10 @@ int launch_sweep_bf16(const SweepPlan &p, const void *in, void *in_next, void *o
 // Enqueue one pass of `sweeps` sweeps over a whole grid (pass.hpp): in_next
 // gets in after that many refreshes.  Only where pass_built.  With sweeps == 0
 // the kernel's code is loaded and nothing launched.
-int launch_pass(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
-int launch_pass_f64(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
-int launch_pass_f32(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
-int launch_pass_bf16(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s);
+int launch_pass(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
+int launch_pass_f64(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
+int launch_pass_f32(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
+int launch_pass_bf16(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
 
 // Sweeps of one pass at most: keeps a launch's time and the loss from an
 // interrupted one bounded (star R=2 FP64 at n = 30000: 256 sweeps take about

@@ -155,7 +155,7 @@ int launch_dtype(const SweepPlan &p, const void *in, void *in_next, void *out, h
 // nothing is launched: the kernel's code is loaded, so that a later launch
 // does not wait for it.
 template <int DT, int P, int R>
-int launch_pass_pr(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
+int launch_pass_pr(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s)
 {
     if constexpr (pass_ok<DT, P, R>()) {
         constexpr int V = SweepGeom<DT, R>::V;
@@ -168,6 +168,7 @@ int launch_pass_pr(const SweepPlan &p, int sweeps, const void *in, void *in_next
         a.nstrips = (p.n + 64 * V - 1) / (64 * V);
         a.rows = pass_rows<DT, P, R>();
         a.sweeps = sweeps;
+        a.any = any;
         const int per_block = a.rows * kWavesPerBlock;
         const unsigned blocks = (unsigned)a.nstrips * (unsigned)((p.n + per_block - 1) / per_block);
         const auto kernel =
@@ -194,25 +195,25 @@ int launch_pass_pr(const SweepPlan &p, int sweeps, const void *in, void *in_next
 }
 
 template <int DT>
-int launch_pass_dtype(const SweepPlan &p, int sweeps, const void *in, void *in_next, void *out, hipStream_t s)
+int launch_pass_dtype(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s)
 {
     switch (p.pattern * 8 + p.radius) {
-    case 1: return launch_pass_pr<DT, STAR, 1>(p, sweeps, in, in_next, out, s);
-    case 2: return launch_pass_pr<DT, STAR, 2>(p, sweeps, in, in_next, out, s);
-    case 3: return launch_pass_pr<DT, STAR, 3>(p, sweeps, in, in_next, out, s);
-    case 4: return launch_pass_pr<DT, STAR, 4>(p, sweeps, in, in_next, out, s);
-    case 5: return launch_pass_pr<DT, STAR, 5>(p, sweeps, in, in_next, out, s);
-    case 6: return launch_pass_pr<DT, STAR, 6>(p, sweeps, in, in_next, out, s);
-    case 7: return launch_pass_pr<DT, STAR, 7>(p, sweeps, in, in_next, out, s);
-    case 8: return launch_pass_pr<DT, STAR, 8>(p, sweeps, in, in_next, out, s);
-    case 9: return launch_pass_pr<DT, GRID, 1>(p, sweeps, in, in_next, out, s);
-    case 10: return launch_pass_pr<DT, GRID, 2>(p, sweeps, in, in_next, out, s);
-    case 11: return launch_pass_pr<DT, GRID, 3>(p, sweeps, in, in_next, out, s);
-    case 12: return launch_pass_pr<DT, GRID, 4>(p, sweeps, in, in_next, out, s);
-    case 13: return launch_pass_pr<DT, GRID, 5>(p, sweeps, in, in_next, out, s);
-    case 14: return launch_pass_pr<DT, GRID, 6>(p, sweeps, in, in_next, out, s);
-    case 15: return launch_pass_pr<DT, GRID, 7>(p, sweeps, in, in_next, out, s);
-    case 16: return launch_pass_pr<DT, GRID, 8>(p, sweeps, in, in_next, out, s);
+    case 1: return launch_pass_pr<DT, STAR, 1>(p, sweeps, any, in, in_next, out, s);
+    case 2: return launch_pass_pr<DT, STAR, 2>(p, sweeps, any, in, in_next, out, s);
+    case 3: return launch_pass_pr<DT, STAR, 3>(p, sweeps, any, in, in_next, out, s);
+    case 4: return launch_pass_pr<DT, STAR, 4>(p, sweeps, any, in, in_next, out, s);
+    case 5: return launch_pass_pr<DT, STAR, 5>(p, sweeps, any, in, in_next, out, s);
+    case 6: return launch_pass_pr<DT, STAR, 6>(p, sweeps, any, in, in_next, out, s);
+    case 7: return launch_pass_pr<DT, STAR, 7>(p, sweeps, any, in, in_next, out, s);
+    case 8: return launch_pass_pr<DT, STAR, 8>(p, sweeps, any, in, in_next, out, s);
+    case 9: return launch_pass_pr<DT, GRID, 1>(p, sweeps, any, in, in_next, out, s);
+    case 10: return launch_pass_pr<DT, GRID, 2>(p, sweeps, any, in, in_next, out, s);
+    case 11: return launch_pass_pr<DT, GRID, 3>(p, sweeps, any, in, in_next, out, s);
+    case 12: return launch_pass_pr<DT, GRID, 4>(p, sweeps, any, in, in_next, out, s);
+    case 13: return launch_pass_pr<DT, GRID, 5>(p, sweeps, any, in, in_next, out, s);
+    case 14: return launch_pass_pr<DT, GRID, 6>(p, sweeps, any, in, in_next, out, s);
+    case 15: return launch_pass_pr<DT, GRID, 7>(p, sweeps, any, in, in_next, out, s);
+    case 16: return launch_pass_pr<DT, GRID, 8>(p, sweeps, any, in, in_next, out, s);
     }
     return set_error(PRK_ENOSTENCIL, "no stencil for pattern %d radius %d", p.pattern, p.radius);
 }

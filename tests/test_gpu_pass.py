@@ -102,3 +102,36 @@ def test_first_run_is_timed_without_loading_code(gpu):
         text = subprocess.run([str(exe), "10", "1000"], capture_output=True, text=True, timeout=60, check=True).stdout
         times.append(float(re.search(r"Avg time \(s\):\s*(\S+)", text).group(1)))
     assert min(times) < 30e-6, times
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("pattern,radius", [(0, 1), (0, 2), (0, 4), (0, 8), (1, 1), (1, 2), (1, 3), (1, 4)])
+def test_run_of_any_values(gpu, pattern, radius, dtype):
+    """An even number of iterations runs sweep 0, which reads the caller's
+    values, inside the pass.  Values whose products with the weights round
+    below the normal range, and sums that lie there themselves, give the bits
+    of sweeps one by one; so do ordinary and large ones, on an out that holds
+    values already."""
+    n = 64 * VEC[dtype] + 13
+    tiny, big = (2.0**-1060, 2.0**900) if dtype == F64 else (2.0**-138, 2.0**100)
+    td = K.torch_dtype(dtype)
+    gen = torch.Generator(device=gpu).manual_seed(9)
+    a, o = (torch.rand((n, n), generator=gen, device=gpu, dtype=torch.float64) * 2 - 1 for _ in range(2))
+    a[: n // 2] *= tiny
+    a[n // 2 + 20 : n // 2 + 24] *= big
+    o[: n // 2] = 0.0
+    for iters in (2, 10):
+        print(f"any p{pattern} r{radius} d{dtype} n={n} iterations={iters}", flush=True)
+        got, want = ([K.alloc_grid(n, dtype) for _ in range(3)] for _ in range(2))
+        for g in (got, want):
+            g[0].copy_(a.to(td))
+            g[1].zero_()
+            g[2].copy_(o.to(td))
+        final, _ = K.run(pattern, radius, dtype, iters, *got)
+        src, dst, out = want
+        for _ in range(iters + 1):
+            K.sweep(pattern, radius, dtype, src, dst, out)
+            src, dst = dst, src
+        assert final == (iters + 1) % 2
+        assert np.array_equal(bits(host(got[2])), bits(host(out))), iters
+        assert np.array_equal(bits(host(got[final])), bits(host(src))), iters
