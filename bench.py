@@ -164,7 +164,9 @@ def config4_solves(seed: int = 7, count: int = 4096):
 def solve_bytes(spec) -> int:
     """Algorithmic bytes of one solve: init writes in and out, each of the
     K+1 fused sweeps reads in, writes in_next, reads and writes the interior
-    of out, the norm reads the interior once."""
+    of out, the norm reads the interior once.  Several sweeps that run in one
+    pass over a grid move less than this, so a rate formed with it
+    (effective_gbs) may exceed HBM's."""
     pattern, radius, dtype, n, iters = spec[:5]
     s = {0: 8, 1: 4, 2: 2}[dtype]
     m = n - 2 * radius
@@ -777,7 +779,7 @@ def fp32_storage_section(a, torch, K, ms_f64: float) -> dict:
 
 def batch_section(a, torch, K) -> dict:
     """The 4096 uneven grids of the batched workload (FP32 storage) in one
-    hipGraph of round launches, against the same solves one grid per launch
+    hipGraph, against the same solves one grid per launch
     in FP64: solves/s of each (after tuning the tile heights unless
     --no-tune; one warm-up run, then three timed runs of the batch)."""
     import numpy as np
