@@ -56,6 +56,14 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 //    empty, against the share of halo rows (FP64 star R=4, n = 2000: 16 rows
 //    are 0.98 of a turn, 25 us; 12 rows 1.3 turns, 32 us; FP64 grid R=5, n =
 //    1000: 8 rows 16 us, 24 rows 44).  Stars and grids of R <= 2 keep 8 rows.
+//  - Where that is no more than one turn, the time is that of one wave going
+//    down its h + 2R rows, and lower tiles are faster until the chip is full:
+//    the lowest that give one workgroup per CU or two, where two on a CU take
+//    9/7 of the time per row of one (BF16, whose rows are longer chains, 12/11
+//    except the stars from R = 6).  8 rows (BF16 12) -> the rule: FP64 star
+//    R=2, n = 150 6.5 -> 3.5 us, n = 512 7.0 -> 4.2, n = 1000 8.3 -> 8.1,
+//    grid R=5, n = 512 14.6 -> 6.9; FP32 star R=2, n = 1000 7.9 -> 5.5; BF16
+//    grid R=3, n = 1000 15.1 -> 8.4, star R=2, n = 2000 10.5 -> 9.2.
 prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
 {
     static const signed char kRows[3][2][kMaxRadius] = {
@@ -93,6 +101,13 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
                 rows = h;
             }
         }
+    }
+    if (tiles(rows) <= turn) {
+        const int cap = (int)((groups * n + turn - 1) / turn), half = (int)((groups * n + turn / 2 - 1) / (turn / 2));
+        const int h2 = std::max(1, cap), h1 = std::max(1, half);
+        const bool slow_rows = d == BF16 && (p == 1 || R <= 5);
+        const int two = slow_rows ? 12 : 9, one = slow_rows ? 11 : 7;
+        rows = std::min(rows, one * (h1 + 2 * R) <= two * (h2 + 2 * R) ? h1 : h2);
     }
     t.rows_per_wave = std::max(1, std::min(rows, n));
     t.gbs = 0.0;

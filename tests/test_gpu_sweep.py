@@ -505,3 +505,37 @@ def test_grid_row_pairs_bitwise(gpu, oracle, radius):
                 assert np.array_equal((b0, b1)[fb].contiguous().cpu().numpy().view(np.uint64), ref_in.view(np.uint64))
     finally:
         K.check(L.prk_set_rows_per_wave(0))
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("pattern,radius", [(0, 1), (0, 5), (0, 8), (1, 2), (1, 3), (1, 8)])
+def test_small_grids_default_height(gpu, pattern, radius, dtype):
+    """The default tile heights of small grids, on either side of the sizes
+    where they change: no more than two workgroups per CU where the height for
+    larger grids gave no more, and the bits of 8-row tiles."""
+    import ctypes
+
+    from kernels_amd._lib import Tuning
+
+    lib = K.lib()
+    lanes = {0: 128, 1: 256, 2: 512}[dtype]
+    for n in (2 * radius + 1, 64, 256, 257, 4 * lanes, 4 * lanes + 1):
+        print(f"height p{pattern} r{radius} d{dtype} n={n}", flush=True)
+        t = Tuning()
+        assert lib.prk_tuning_get(pattern, radius, dtype, n, ctypes.byref(t)) == 0
+        groups = -(-(-(-n // lanes)) // 4)
+        assert 1 <= t.rows_per_wave <= 48
+        if n <= 1024:
+            assert groups * -(-n // t.rows_per_wave) <= 512
+        results = []
+        for rows in (0, 8):
+            a, b, out = (K.alloc_grid(n, dtype) for _ in range(3))
+            K.init(K.INIT_SEEDED, 5, dtype, a, out)
+            lib.prk_set_rows_per_wave(rows)
+            try:
+                K.sweep(pattern, radius, dtype, a, b, out)
+                K.stencil_ex(pattern, radius, dtype, b, out)
+            finally:
+                lib.prk_set_rows_per_wave(0)
+            results.append((b.clone(), out.clone()))
+        assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
