@@ -75,6 +75,7 @@ struct Round {
 using namespace prk;
 
 struct prk_batch {
+    int device = 0;  // that holds the grids
     std::vector<prk_solve> solves;
     std::vector<BGrid> grids;  // host copies
     void *pool = nullptr;      // grids
@@ -117,6 +118,21 @@ int validate_solve(const prk_solve &s)
     if (s.init != PRK_INIT_ANALYTIC && s.init != PRK_INIT_SEEDED) return set_error(PRK_EINVAL, "bad init");
     return PRK_OK;
 }
+
+// Makes `device` the calling thread's current one until it goes out of scope.
+struct DeviceScope {
+    int before = 0, rc;
+    explicit DeviceScope(int device)
+    {
+        rc = check_hip(hipGetDevice(&before), "hipGetDevice");
+        if (!rc && device != before) rc = check_hip(hipSetDevice(device), "hipSetDevice");
+    }
+    ~DeviceScope()
+    {
+        int now = 0;
+        if (hipGetDevice(&now) == hipSuccess && now != before) (void)hipSetDevice(before);
+    }
+};
 
 // Workgroup entries of one stage of solve g.
 void push_work(std::vector<RWork> &work, Round &r, const BGrid &bg, int g, int stage)
@@ -378,7 +394,10 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
     for (int i = 0; i < count; ++i)
         if ((rc = validate_solve(solves[i]))) return rc;
 
+    int device = 0;
+    if ((rc = check_hip(hipGetDevice(&device), "hipGetDevice"))) return rc;
     prk_batch *b = new prk_batch();
+    b->device = device;
     b->solves.assign(solves, solves + count);
     b->grids.resize(count);
 
@@ -564,7 +583,10 @@ int prk_batch_output(const prk_batch *b, int idx, int which, void *host, size_t 
     // A copy of rows with a pitch moves them one by one, about 7 us each on
     // MI355X (n = 1000 FP32: 6.9 ms), so the rows are packed on the device
     // first, in the order the copy itself would have (the null stream), and
-    // move as one block (0.23 ms).
+    // move as one block (0.23 ms).  The calling thread may have another
+    // device current than the one that holds the grids.
+    const DeviceScope on(b->device);
+    if (on.rc) return on.rc;
     const void *dense = g.pitch == g.n ? src : nullptr;
     std::unique_lock<std::mutex> lock(b->pack_mu, std::defer_lock);
     if (!dense) {

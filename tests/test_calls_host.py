@@ -1,0 +1,90 @@
+"""What calls of the library ask of the HIP runtime, on the CPU: the host code
+built without device code against a stand-in (tests/host/mock_calls.cc) that
+records launches."""
+import ctypes as C
+import os
+import shutil
+import subprocess
+import threading
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+SOURCES = [ROOT / "kernels_amd/csrc" / f for f in ("prk_api.hip", "batch.hip", "autotune.hip")]
+SOURCES.append(ROOT / "tests/host/mock_calls.cc")
+
+pytestmark = pytest.mark.skipif(not (os.path.exists(HIPCC) and SOURCES[-1].exists()), reason="needs hipcc")
+
+
+class Solve(C.Structure):
+    _fields_ = [(f, C.c_int) for f in ("pattern", "radius", "dtype", "n", "iterations", "init")] + [
+        ("seed", C.c_uint64)]
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("calls")
+
+    def compile_one(src):
+        obj = tmp / (src.name + ".o")
+        subprocess.run([HIPCC, "--offload-host-only", "-O1", "-std=c++17", "-fPIC", f"-I{ROOT / 'include'}",
+                        f"-I{ROOT / 'kernels_amd/csrc'}", "-x", "hip", "-c", str(src), "-o", str(obj)],
+                       check=True, capture_output=True, text=True)
+        return str(obj)
+
+    objs = [compile_one(s) for s in SOURCES]
+    # the device code that the host code would register does not exist here
+    names = subprocess.run(["nm", "-u", *objs], check=True, capture_output=True, text=True).stdout.split()
+    defs = [f"-Wl,--defsym={s}=0" for s in sorted(set(names)) if s.startswith("__hip_fatbin")]
+    so = tmp / "libcalls.so"
+    subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-o", str(so), *objs, *defs, "-lpthread"], check=True, capture_output=True,
+                   text=True)
+    L = C.CDLL(str(so))
+    L.prk_last_error.restype = C.c_char_p
+    L.mock_reset()
+    return L
+
+
+def check(L, rc):
+    assert rc == 0, L.prk_last_error()
+
+
+def kernels(L):
+    v = (C.c_uint * 3)()
+    out = []
+    for i in range(L.mock_kernels()):
+        L.mock_kernel(i, v)
+        out.append(tuple(v))
+    return out
+
+
+def test_batch_output_runs_on_the_batch_s_device(lib):
+    # the thread that fetches a grid has another device current than the one
+    # the batch was made on: the rows are packed where they lie, and the
+    # thread's device is as it was
+    L, n = lib, 100
+    batch = C.c_void_p()
+    L.hipSetDevice(1)
+    try:
+        check(L, L.prk_batch_create(C.byref(Solve(0, 1, 1, n, 2, 1, 5)), 1, 0, 0, C.byref(batch)))
+    finally:
+        L.hipSetDevice(0)
+    before = L.mock_bytes_on(0)
+    seen = []
+
+    def fetch():
+        host = np.zeros((n, n), np.float32)
+        L.mock_reset()
+        rc = L.prk_batch_output(batch, 0, 0, host.ctypes.data_as(C.c_void_p), C.c_size_t(host.nbytes))
+        dev = C.c_int(-1)
+        L.hipGetDevice(C.byref(dev))
+        seen.extend([rc, dev.value, [k[2] for k in kernels(L)]])
+
+    t = threading.Thread(target=fetch)
+    t.start()
+    t.join()
+    assert seen == [0, 0, [1]] and L.mock_bytes_on(0) == before
+    L.prk_batch_destroy(batch)
