@@ -82,10 +82,10 @@ int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const
     plan->span = whole_grid(n);
     plan->pitch = pitch;
     plan->pad_writable = false;
-    plan->mode = ptrs % 4 != 0                ? MODE_ELEM
-                 : ptrs % 16 != 0             ? MODE_DWORD
-                 : n % vec_width(dtype) != 0 ? MODE_RAGGED
-                                              : MODE_VEC;
+    const bool short_rows = (unsigned long long)n * es < 16;  // MODE_DWORD reads up to 16 bytes of the next row
+    plan->mode = ptrs % 16 == 0                 ? (n % vec_width(dtype) != 0 ? MODE_RAGGED : MODE_VEC)
+                 : ptrs % 4 != 0 || short_rows ? MODE_ELEM
+                                                : MODE_DWORD;
     const prk_tuning t = choose_tuning(pattern, radius, dtype, n);
     plan->variant = g_variant_override >= 0 ? g_variant_override : t.variant;
     plan->order = g_order >= 0 ? g_order : t.order;

@@ -769,7 +769,9 @@ __device__ inline void bstore_elem(__amdgpu_buffer_rsrc_t r, unsigned off, T v)
 //               needs no more), but a row's last vector may run past the row.
 //               The bytes behind it are the next row's, so it is loaded whole
 //               there too; only the array's last row is read by element.
-//   MODE_ELEM   element loads and stores (BF16 rows on odd elements).
+//               Rows of 16 bytes or more: the vector must end in the next row.
+//   MODE_ELEM   element loads and stores (BF16 rows on odd elements, rows of
+//               under 16 bytes).
 // Measured on MI355X, element accesses -> these: fused sweeps at n=9999, rows
 // on 128 bytes, FP32 star R=1 421 -> 274 us (n=10000: 274), FP64 star R=2
 // 640 -> 536, BF16 grid R=3 331 -> 167; at n=4001, pitch 4001, FP64 star R=2
@@ -791,9 +793,10 @@ __device__ inline u32x4 load_row_vec(__amdgpu_buffer_rsrc_t r, unsigned off, boo
 
 // Byte range of the resource a row is loaded through.
 template <int MODE>
-__device__ inline unsigned row_load_bytes(unsigned row_bytes, bool end)
+__host__ __device__ inline unsigned row_load_bytes(unsigned row_bytes, bool end)
 {
-    return MODE == MODE_DWORD && !end ? min(row_bytes + 16u, kOOB) : row_bytes;
+    if (MODE != MODE_DWORD || end) return row_bytes;
+    return row_bytes + 16u < kOOB ? row_bytes + 16u : kOOB;
 }
 
 // One vector of in_next at byte offset off (kOOB: none); `ragged`: the wave

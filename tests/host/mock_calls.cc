@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "prk_internal.hpp"
+#include "sweep.hpp"
 
 using namespace prk;
 
@@ -29,7 +30,8 @@ std::mutex g_mu;
 std::map<const char *, Alloc> g_allocs;
 std::vector<Kernel> g_kernels;
 struct Sweeps {
-    int sweeps, any, rows, wgs, mode;
+    int sweeps, any, rows, wgs;
+    long long reach;  // bytes from the grid's start to the end of what a row before the last loads
     const void *in, *in_next;
 };
 std::vector<Sweeps> g_sweeps;  // launch_sweep (sweeps = 1, any = -1) and launch_pass calls
@@ -46,8 +48,11 @@ struct Stream {
 
 int record(const SweepPlan &p, int sweeps, int any, const void *in, const void *in_next)
 {
+    const unsigned row_bytes = (unsigned)(p.pitch * (long long)dtype_size(p.dtype));
+    const unsigned load = p.mode == MODE_DWORD ? row_load_bytes<MODE_DWORD>(row_bytes, false) : row_bytes;
     std::lock_guard<std::mutex> l(g_mu);
-    g_sweeps.push_back(Sweeps{sweeps, any, p.rows_per_wave, p.wgs_per_cu, p.mode, in, in_next});
+    g_sweeps.push_back(Sweeps{sweeps, any, p.rows_per_wave, p.wgs_per_cu, (long long)(p.span.nrows - 2) * row_bytes + load,
+                              in, in_next});
     return 0;
 }
 }  // namespace
@@ -86,7 +91,7 @@ int mock_sweeps(void) { return (int)g_sweeps.size(); }
 void mock_sweep(int i, long long *v)
 {
     const Sweeps &s = g_sweeps[i];
-    const long long x[] = {s.sweeps, s.any, s.rows, s.wgs, s.mode, (long long)s.in, (long long)s.in_next};
+    const long long x[] = {s.sweeps, s.any, s.rows, s.wgs, s.reach, (long long)s.in, (long long)s.in_next};
     std::memcpy(v, x, sizeof x);
 }
 int mock_bytes_on(int device)  // MiB allocated there

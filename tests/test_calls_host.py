@@ -61,6 +61,16 @@ def kernels(L):
     return out
 
 
+def sweeps(L):
+    """(sweeps, any, rows, workgroups per CU, reach, in, in_next) of each launch."""
+    v = (C.c_longlong * 7)()
+    out = []
+    for i in range(L.mock_sweeps()):
+        L.mock_sweep(i, v)
+        out.append(tuple(v))
+    return out
+
+
 def test_batch_output_runs_on_the_batch_s_device(lib):
     # the thread that fetches a grid has another device current than the one
     # the batch was made on: the rows are packed where they lie, and the
@@ -88,3 +98,18 @@ def test_batch_output_runs_on_the_batch_s_device(lib):
     t.join()
     assert seen == [0, 0, [1]] and L.mock_bytes_on(0) == before
     L.prk_batch_destroy(batch)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_sweep_reads_stay_inside_the_grid(lib, dtype):
+    # rows off 16-byte boundaries are read in vectors that may run past their
+    # row; a row before the last must not read past the last one's elements
+    L, es = lib, (8, 4, 2)[dtype]
+    for n in range(3, 20):
+        for pitch in range(n, n + 9):
+            for offset in (0, 4, 8):
+                p = [C.c_void_p((k << 20) + offset) for k in (1, 2, 3)]
+                L.mock_reset()
+                check(L, L.prk_sweep(0, 1, dtype, n, C.c_longlong(pitch), *p, None))
+                (s,) = sweeps(L)
+                assert s[4] <= ((n - 1) * pitch + n) * es, (n, pitch, offset)
