@@ -172,11 +172,15 @@ __global__ __launch_bounds__(256) void add_one_flat_kernel(void *buf, long long 
     }
 }
 
+static long long add_flat_threads(int dtype, long long count)
+{
+    return count / vec_width(dtype) + count % vec_width(dtype);
+}
+
 template <int DT>
 static int launch_add_flat(long long count, void *in, hipStream_t s)
 {
-    constexpr int V = DTypeTraits<DT>::V;
-    const long long threads = count / V + count % V;
+    const long long threads = add_flat_threads(DT, count);
     const dim3 blocks((unsigned)((threads + 255) / 256));
     const bool nt = count * (long long)sizeof(typename DTypeTraits<DT>::T) > kLastLevelCache;
     if (nt) hipLaunchKernelGGL((add_one_flat_kernel<DT, true>), blocks, dim3(256), 0, s, in, count);
@@ -190,8 +194,10 @@ static int launch_add(int dtype, int n, long long pitch, void *in, hipStream_t s
     if (n < 1 || pitch < n || !in) return set_error(PRK_EINVAL, "bad grid (n=%d pitch=%lld)", n, pitch);
     const bool vec = ((uintptr_t)in % 16 == 0) && ((pitch * dtype_size(dtype)) % 16 == 0);
     const int V = vec_width(dtype);
-    if (pitch == n && (uintptr_t)in % 16 == 0) {
-        const long long count = (long long)n * n;
+    // A launch holds fewer than 2^32 threads: larger grids (FP64 from n =
+    // 92682 on) go row by row, which has a bounded launch.
+    const long long count = (long long)n * n;
+    if (pitch == n && (uintptr_t)in % 16 == 0 && add_flat_threads(dtype, count) <= (1ll << 32) - 256) {
         return dtype == F64 ? launch_add_flat<F64>(count, in, s)
                : dtype == F32 ? launch_add_flat<F32>(count, in, s)
                               : launch_add_flat<BF16>(count, in, s);

@@ -113,3 +113,12 @@ def test_sweep_reads_stay_inside_the_grid(lib, dtype):
                 check(L, L.prk_sweep(0, 1, dtype, n, C.c_longlong(pitch), *p, None))
                 (s,) = sweeps(L)
                 assert s[4] <= ((n - 1) * pitch + n) * es, (n, pitch, offset)
+
+
+@pytest.mark.parametrize("dtype,n", [(0, 92680), (0, 92681), (0, 92682), (0, 130001), (1, 131071), (1, 131072),
+                                     (2, 185363), (2, 185364), (2, 300000)])
+def test_add_of_very_large_grids_is_launched(lib, dtype, n):
+    # a launch holds fewer than 2^32 threads: larger dense grids go row by row
+    lib.mock_reset()
+    check(lib, lib.prk_add_ex(dtype, n, C.c_longlong(n), C.c_void_p(1 << 20), None))
+    assert len(kernels(lib)) == 1
