@@ -37,7 +37,10 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 
 }  // namespace
 
-// Measured defaults on MI355X: a 3-row non-temporal pipeline, and by size:
+// Measured defaults on MI355X: a 3-row non-temporal pipeline, and by size (of
+// a slab: the grid's n, and its own rows where turns of the chip are counted;
+// by the whole grid's tiles FP32 star R=3, n = 3001, one of eight slabs took
+// 16.2 us instead of 8.0):
 //  - Large grids take the row blocks and workgroups per CU that were fastest
 //    at n = 16384 for each stencil: the HBM-bound sweeps want two workgroups
 //    per CU, those with longer row steps as many as fit.  Against the rule
@@ -64,7 +67,7 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 //    R=2, n = 150 6.5 -> 3.5 us, n = 512 7.0 -> 4.2, n = 1000 8.3 -> 8.1,
 //    grid R=5, n = 512 14.6 -> 6.9; FP32 star R=2, n = 1000 7.9 -> 5.5; BF16
 //    grid R=3, n = 1000 15.1 -> 8.4, star R=2, n = 2000 10.5 -> 9.2.
-prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
+prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n, int nrows)
 {
     static const signed char kRows[3][2][kMaxRadius] = {
         {{8, 8, 12, 12, 8, 8, 12, 24}, {8, 8, 12, 24, 32, 48, 48, 32}},
@@ -88,7 +91,7 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
     }
     const int lanes = d == F64 ? 128 : d == F32 ? 256 : 512;  // columns of a strip
     const long long groups = ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock, turn = 512;
-    auto tiles = [&](int h) { return groups * ((n + h - 1) / h); };
+    auto tiles = [&](int h) { return groups * ((nrows + h - 1) / h); };
     if ((R >= 3 || d == BF16) && tiles(rows) < (d == BF16 ? 2 : 3) * turn) {
         static const int kHeights[] = {8, 12, 16, 24, 32};
         double best = 0.0;
@@ -103,7 +106,7 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
         }
     }
     if (tiles(rows) <= turn) {
-        const int cap = (int)((groups * n + turn - 1) / turn), half = (int)((groups * n + turn / 2 - 1) / (turn / 2));
+        const int cap = (int)((groups * nrows + turn - 1) / turn), half = (int)((groups * nrows + turn / 2 - 1) / (turn / 2));
         const int h2 = std::max(1, cap), h1 = std::max(1, half);
         const bool slow_rows = d == BF16 && (p == 1 || R <= 5);
         const int two = slow_rows ? 12 : 9, one = slow_rows ? 11 : 7;
@@ -114,7 +117,7 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n)
     return t;
 }
 
-prk_tuning choose_tuning(int pattern, int radius, int dtype, int n)
+prk_tuning choose_tuning(int pattern, int radius, int dtype, int n, int nrows)
 {
     {
         std::lock_guard<std::mutex> lock(g_mu);
@@ -139,7 +142,7 @@ prk_tuning choose_tuning(int pattern, int radius, int dtype, int n)
             return t;
         }
     }
-    return heuristic_tuning(pattern, radius, dtype, n);
+    return heuristic_tuning(pattern, radius, dtype, n, nrows);
 }
 
 }  // namespace prk
@@ -151,7 +154,7 @@ extern "C" {
 int prk_tuning_get(int pattern, int radius, int dtype, int n, prk_tuning *t)
 {
     if (!t) return set_error(PRK_EINVAL, "null tuning");
-    *t = choose_tuning(pattern, radius, dtype, n);
+    *t = choose_tuning(pattern, radius, dtype, n, n);
     return PRK_OK;
 }
 

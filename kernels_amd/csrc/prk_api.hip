@@ -55,7 +55,7 @@ static bool valid_dtype(int dt) { return dt == F64 || dt == F32 || dt == BF16; }
 static int vec_width(int dt) { return dt == F64 ? 2 : dt == F32 ? 4 : 8; }
 
 int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const void *in,
-               const void *in_next, const void *out, int rows_per_wave, SweepPlan *plan)
+               const void *in_next, const void *out, int rows_per_wave, SweepPlan *plan, int nrows)
 {
     if (pattern != STAR && pattern != GRID)
         return set_error(PRK_EINVAL, "pattern must be 0 (star) or 1 (grid), got %d", pattern);
@@ -86,7 +86,7 @@ int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const
     plan->mode = ptrs % 16 == 0                 ? (n % vec_width(dtype) != 0 ? MODE_RAGGED : MODE_VEC)
                  : ptrs % 4 != 0 || short_rows ? MODE_ELEM
                                                 : MODE_DWORD;
-    const prk_tuning t = choose_tuning(pattern, radius, dtype, n);
+    const prk_tuning t = choose_tuning(pattern, radius, dtype, n, nrows > 0 ? nrows : n);
     plan->variant = g_variant_override >= 0 ? g_variant_override : t.variant;
     plan->order = g_order >= 0 ? g_order : t.order;
     plan->wgs_per_cu = g_wgs_per_cu >= 0 ? g_wgs_per_cu : t.wgs_per_cu;
@@ -680,17 +680,18 @@ int prk_sweep_slab(int pattern, int radius, int dtype, int n, int row0, int rows
                    const void *in, void *in_next, void *out, void *stream)
 {
     if (!in_next) return set_error(PRK_EINVAL, "fused sweep needs in_next");
+    const bool inside = row0 >= 0 && rows >= 1 && row0 < n && rows <= n - row0;
+    const int top = inside ? std::min(radius, row0) : 0, bot = inside ? std::min(radius, n - row0 - rows) : 0;
     SweepPlan p;
-    int rc = plan_sweep(pattern, radius, dtype, n, pitch, in, in_next, out, 0, &p);
+    int rc = plan_sweep(pattern, radius, dtype, n, pitch, in, in_next, out, 0, &p, inside ? top + rows + bot : 0);
     if (rc) return rc;
-    if (row0 < 0 || rows < 1 || rows > n - row0)
+    if (!inside)
         return set_error(PRK_EINVAL, "slab of rows [%d, %lld) is not inside the %d rows of the grid", row0,
                          (long long)row0 + rows, n);
     // Local row 0 is global row row0 - top.  The first R local rows are halo
     // rows or frame rows (top < R only when row0 < R), and so are the last R,
     // so the outputs, global rows [max(row0, R), min(row0+rows, n-R)), are
     // local rows [R, nrows-R) as for a whole grid (empty when nrows < 2R+1).
-    const int top = std::min(radius, row0), bot = std::min(radius, n - row0 - rows);
     p.span.nrows = top + rows + bot;
     p.span.upd_lo = top;
     p.span.upd_hi = top + rows;

@@ -49,13 +49,14 @@ int l1norm_async(int dtype, int n, long long pitch, int radius, const void *out,
                  hipStream_t s);
 
 // Tiling a sweep of this shape uses: tuned entry, nearest tuned size, or the
-// built-in default (autotune.hip).
-prk_tuning choose_tuning(int pattern, int radius, int dtype, int n);
-prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n);
+// built-in default (autotune.hip).  nrows: rows of the array, n of a whole grid.
+prk_tuning choose_tuning(int pattern, int radius, int dtype, int n, int nrows);
+prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n, int nrows);
 
-// Fills the launch geometry; rows_per_wave <= 0 picks automatically.
+// Fills the launch geometry; rows_per_wave <= 0 picks automatically, for an
+// array of nrows rows (0: a whole grid).
 int plan_sweep(int pattern, int radius, int dtype, int n, long long pitch, const void *in,
-               const void *in_next, const void *out, int rows_per_wave, SweepPlan *plan);
+               const void *in_next, const void *out, int rows_per_wave, SweepPlan *plan, int nrows = 0);
 
 // Enqueue one sweep (in_next == nullptr: unfused).
 int launch_sweep(const SweepPlan &p, const void *in, void *in_next, void *out, hipStream_t s);

@@ -122,3 +122,17 @@ def test_add_of_very_large_grids_is_launched(lib, dtype, n):
     lib.mock_reset()
     check(lib, lib.prk_add_ex(dtype, n, C.c_longlong(n), C.c_void_p(1 << 20), None))
     assert len(kernels(lib)) == 1
+
+
+@pytest.mark.parametrize("n,least", [(1000, 128), (2000, 256), (3001, 256)])
+def test_tiles_of_a_small_slab_fill_the_chip(lib, n, least):
+    # the height goes by the slab's own rows: an eighth of a grid's rows in
+    # tiles chosen for the whole grid left most of the 256 CUs idle
+    L, rows = lib, n // 8
+    p = [C.c_void_p(k << 30) for k in (1, 2, 3)]
+    L.mock_reset()
+    pitch = C.c_longlong((n + 15) // 16 * 16)
+    check(L, L.prk_sweep_slab(0, 2, 0, n, 3 * rows, rows, pitch, *p, None))
+    (s,) = sweeps(L)
+    groups = ((n + 127) // 128 + 3) // 4
+    assert groups * -(-(rows + 4) // s[2]) >= least
