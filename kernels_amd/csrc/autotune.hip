@@ -37,44 +37,58 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 
 }  // namespace
 
-// Measured defaults on MI355X: a 3-row non-temporal pipeline, and by size (of
-// a slab: the grid's n, and its own rows where turns of the chip are counted;
-// by the whole grid's tiles FP32 star R=3, n = 3001, one of eight slabs took
-// 16.2 us instead of 8.0):
-//  - Large grids take the row blocks and workgroups per CU that were fastest
-//    at n = 16384 for each stencil: the HBM-bound sweeps want two workgroups
-//    per CU, those with longer row steps as many as fit.  Against the rule
-//    below for the middle: FP64 star R=8 1683 -> 1547 us; FP32 star R=5 797
-//    -> 730, grid R=5 1010 -> 901; BF16 star R=1 404 -> 380, grid R=6 942 ->
-//    853.  The FP64 grids from R = 3 and the FP32 grid R=5, which are bound
-//    by their arithmetic, take theirs at every size (FP64 grid R=5, n = 5000:
-//    272 -> 213).
+// Measured defaults on MI355X: a 3-row non-temporal pipeline, and by size (a
+// slab's turns of the chip counted by its own rows: by the whole grid's, FP32
+// star R=3, n = 3001, one of eight slabs took 16.2 us instead of 8.0):
+//  - Large whole grids take the row blocks and workgroups per CU that were
+//    fastest at n = 16384 for each stencil and no slower anywhere above the
+//    line: the HBM-bound sweeps want two workgroups per CU, those with longer
+//    row steps as many as fit.  Slabs of as many points take them from R = 6
+//    on (BF16 star R=8, n = 22000, half of the rows: 471 -> 414 us), the
+//    others lose (FP32 star R=5 641 -> 670), as do those of fewer points (BF16
+//    grid R=7, n = 18000, an eighth: 198 -> 236; not the FP64 star R=8, whose
+//    height is the same, n = 8504, an eighth: 69 -> 55).  Against the rule
+//    below for the middle: FP64 star R=8 1683 -> 1547 us; FP32 star R=5 797 ->
+//    730, grid R=5 1010 -> 901; BF16 star R=1 404 -> 380, grid R=6 942 -> 853.
+//    Stencils whose best at 16384 lost elsewhere keep the middle's (FP64 star
+//    R=5, 8 rows and four workgroups: n = 10000 484 -> 465 us, but 11000 684
+//    -> 723, 27000 4103 -> 4291).  The FP64 grids of R = 3..7 and the FP32
+//    grid R=5, which are bound by their arithmetic, take theirs at every size
+//    (FP64 grid R=5, n = 5000: 272 -> 213).
 //  - In the middle one height per radius, growing so that the 2R halo rows
 //    each block re-reads stay a small share, and two workgroups per CU (four
 //    in BF16): what was fastest at 16384 loses up to 15 % between 2000 and
-//    8000, where the turns of the chip count (FP64 star R=5, n = 6000: 203
-//    us, 8 rows 220).
-//  - A grid of less than three (BF16: two) turns of two workgroups per CU takes the
-//    height that fills its turns best, the last one of which may be nearly
-//    empty, against the share of halo rows (FP64 star R=4, n = 2000: 16 rows
-//    are 0.98 of a turn, 25 us; 12 rows 1.3 turns, 32 us; FP64 grid R=5, n =
-//    1000: 8 rows 16 us, 24 rows 44).  Stars and grids of R <= 2 keep 8 rows.
+//    8000, where the turns of the chip count (FP64 star R=5, n = 6000: 203 us,
+//    8 rows 220).
+//  - An array of more than one and less than three (BF16: two) turns of two
+//    workgroups per CU takes the height that fills its turns best, the last
+//    one of which may be nearly empty, against the share of halo rows (FP64
+//    grid R=5, n = 4000: 24 rows 222 us, 32 rows 158; the FP32 grid R=5, four
+//    workgroups per CU, keeps its 32: n = 4800 76 us, 24 rows 90).  The
+//    middle's height stays unless another fills the turns clearly better, a
+//    lower one much better (FP64 star R=8, n = 2800: 24 rows 63.9 us, 12 rows,
+//    by this measure 14 % better, 65.5), and where only a few workgroups lie
+//    past two turns (FP32: one), which cost nothing (FP32 grid R=6, n = 7000,
+//    half of the rows, 1029 workgroups of 24 rows: 111 us, one and a half
+//    turns of 32 rows 135).  Stars and grids of R <= 2 keep 8 rows.
 //  - Where that is no more than one turn, the time is that of one wave going
 //    down its h + 2R rows, and lower tiles are faster until the chip is full:
-//    the lowest that give one workgroup per CU or two, where two on a CU take
-//    9/7 of the time per row of one (BF16, whose rows are longer chains, 12/11
-//    except the stars from R = 6).  8 rows (BF16 12) -> the rule: FP64 star
-//    R=2, n = 150 6.5 -> 3.5 us, n = 512 7.0 -> 4.2, n = 1000 8.3 -> 8.1,
-//    grid R=5, n = 512 14.6 -> 6.9; FP32 star R=2, n = 1000 7.9 -> 5.5; BF16
-//    grid R=3, n = 1000 15.1 -> 8.4, star R=2, n = 2000 10.5 -> 9.2.
+//    the lowest that give one workgroup per CU or two.  Two on a CU take 9/7
+//    of the time per row of one; less where a row is one long chain of
+//    arithmetic, which a second wave hides (medians over n = 300..3000: BF16
+//    star R=3 1.19, FP32 grid R=4 1.14, BF16 grid R=3 1.13, star R=5 1.11,
+//    FP32 grid R=6 1.03, FP64 grid R=8 1.07).  8 rows (BF16 12) -> the rule:
+//    FP64 star R=2, n = 150 6.5 -> 3.5 us, n = 512 7.0 -> 4.2, n = 1000 8.3 ->
+//    8.1, grid R=5, n = 512 14.6 -> 6.9; FP32 star R=2, n = 1000 7.9 -> 5.5;
+//    BF16 grid R=3, n = 1000 15.1 -> 8.4, star R=2, n = 2000 10.5 -> 9.2.
 prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n, int nrows)
 {
     static const signed char kRows[3][2][kMaxRadius] = {
-        {{8, 8, 12, 12, 8, 8, 12, 24}, {8, 8, 12, 24, 32, 48, 48, 32}},
-        {{8, 8, 12, 12, 12, 12, 16, 16}, {8, 8, 12, 16, 32, 48, 48, 48}},
+        {{8, 8, 12, 16, 24, 24, 12, 24}, {8, 8, 12, 24, 32, 48, 48, 24}},
+        {{8, 8, 12, 12, 12, 24, 24, 24}, {8, 8, 12, 16, 32, 48, 48, 48}},
         {{8, 8, 12, 12, 12, 12, 24, 24}, {12, 12, 12, 32, 32, 32, 32, 32}}};
     static const signed char kWgs[3][2][kMaxRadius] = {
-        {{2, 2, 2, 2, 4, 4, 4, 4}, {2, 2, 4, 4, 4, 4, 4, 4}},
+        {{2, 2, 2, 2, 2, 2, 4, 4}, {2, 2, 4, 4, 4, 4, 4, 2}},
         {{2, 2, 2, 2, 2, 2, 2, 2}, {2, 2, 2, 2, 4, 4, 4, 4}},
         {{2, 2, 2, 4, 4, 4, 4, 4}, {2, 3, 4, 4, 4, 4, 4, 4}}};
     const int d = dtype == F32 || dtype == BF16 ? dtype : F64, p = pattern == GRID ? 1 : 0;
@@ -84,32 +98,55 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n, int nrows
     t.order = 1;
     int rows = d == BF16 ? 12 : R <= 2 ? 8 : R == 3 ? 12 : R == 4 ? 16 : 24;
     t.wgs_per_cu = d == BF16 ? 4 : 2;
-    const bool large = n >= (d == F64 ? 8000 : 12000);
-    if (large || (p == 1 && ((d == F64 && R >= 3) || (d == F32 && R == 5)))) {
+    // BF16 sweeps of R <= 3 lose by theirs below 16000 (grid R=2, n = 15000:
+    // 332 -> 349 us; 18000 485 -> 461), the wider ones gain from 12000 on.
+    const int line = d == F64 ? 8000 : d == BF16 && R <= 3 ? 16000 : 12000;
+    const bool arithmetic = p == 1 && ((d == F64 && R >= 3 && R <= 7) || (d == F32 && R == 5));
+    const bool wgs_alone = d == F64 && p == 0 && R == 8 && n >= line;  // the middle's height
+    const bool large = wgs_alone || ((long long)n * nrows >= (long long)line * line && (nrows == n || R >= 6));
+    if (large || arithmetic) {
         rows = kRows[d][p][R - 1];
         t.wgs_per_cu = kWgs[d][p][R - 1];
     }
     const int lanes = d == F64 ? 128 : d == F32 ? 256 : 512;  // columns of a strip
-    const long long groups = ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock, turn = 512;
+    constexpr long long kTurn = 512;  // workgroups
+    const long long groups = std::max(1, ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock);
     auto tiles = [&](int h) { return groups * ((nrows + h - 1) / h); };
-    if ((R >= 3 || d == BF16) && tiles(rows) < (d == BF16 ? 2 : 3) * turn) {
+    // a second workgroup on a CU adds nothing to the FP64 grid R=8, and the
+    // FP32 grid R=5 has four
+    const long long lap = d == F64 && p == 1 && R == 8 ? kTurn / 2 : kTurn;
+    const long long over = (tiles(rows) - 1) % lap + 1;  // workgroups of the last turn
+    const bool whole_turns = over <= 12 && (d == F32 || tiles(rows) > 2 * kTurn);
+    if ((R >= 3 || d == BF16) && tiles(rows) > kTurn && tiles(rows) < (d == BF16 ? 2 : 3) * kTurn && !whole_turns &&
+        !(arithmetic && d == F32)) {
         static const int kHeights[] = {8, 12, 16, 24, 32};
+        auto score = [&](int h) {  // share of its turns that the grid fills, times the share of rows that are no halo
+            const long long t = tiles(h), turns = (t + lap - 1) / lap;
+            return (double)t / (double)(turns * lap) * h / (h + 0.6 * R);
+        };
+        const int middle = rows;
+        const double stay = score(middle);
         double best = 0.0;
         for (int h : kHeights) {
             if (d == BF16 && h > 16) break;  // its row steps are long: 24 and 32 rows lose however they fill
-            const long long turns = (tiles(h) + turn - 1) / turn;
-            const double score = (double)tiles(h) / (double)(turns * turn) * h / (h + 0.6 * R);
-            if (score > best) {
-                best = score;
+            if (!arithmetic && score(h) < (h < middle ? 1.25 : h > middle ? 1.05 : 1.0) * stay) continue;
+            if (score(h) > best) {
+                best = score(h);
                 rows = h;
             }
         }
     }
-    if (tiles(rows) <= turn) {
-        const int cap = (int)((groups * nrows + turn - 1) / turn), half = (int)((groups * nrows + turn / 2 - 1) / (turn / 2));
-        const int h2 = std::max(1, cap), h1 = std::max(1, half);
-        const bool slow_rows = d == BF16 && (p == 1 || R <= 5);
-        const int two = slow_rows ? 12 : 9, one = slow_rows ? 11 : 7;
+    if (tiles(rows) <= kTurn) {
+        auto lowest = [&](long long wgs) {  // height of at most that many workgroups, or of one tile per group
+            const long long blocks = std::max(1ll, wgs / groups);
+            return (int)((nrows + blocks - 1) / blocks);
+        };
+        const int h2 = lowest(kTurn), h1 = lowest(kTurn / 2);
+        const bool chains = p == 1 && R >= (d == F64 ? 8 : d == F32 ? 5 : 4);
+        int two = 9, one = 7;
+        if (chains) two = 20, one = 19;
+        else if (d == BF16 && R >= 2 && (p == 1 || (R >= 3 && R <= 5))) two = 12, one = 11;
+        else if ((d == BF16 && p == 0 && R == 2) || (d == F32 && p == 1 && R == 4)) two = 8, one = 7;
         rows = std::min(rows, one * (h1 + 2 * R) <= two * (h2 + 2 * R) ? h1 : h2);
     }
     t.rows_per_wave = std::max(1, std::min(rows, n));

@@ -136,3 +136,30 @@ def test_tiles_of_a_small_slab_fill_the_chip(lib, n, least):
     (s,) = sweeps(L)
     groups = ((n + 127) // 128 + 3) // 4
     assert groups * -(-(rows + 4) // s[2]) >= least
+
+
+class Tuning(C.Structure):
+    _fields_ = [(f, C.c_int) for f in ("variant", "rows_per_wave", "wgs_per_cu", "order")] + [("gbs", C.c_double)]
+
+
+@pytest.mark.parametrize("pattern,radius,dtype,n,rows,wgs", [
+    (1, 8, 0, 3600, 24, 2), (1, 8, 0, 5400, 24, 2),      # 32 rows: 282 -> 300 us, 542 -> 573
+    (0, 4, 0, 18000, 16, 2), (0, 5, 0, 11000, 24, 2), (0, 6, 0, 14000, 24, 2),
+    (0, 8, 0, 2800, 24, 2), (0, 4, 1, 4200, 16, 2), (0, 8, 1, 15000, 24, 2),
+    (1, 2, 2, 15000, 12, 4), (1, 2, 2, 18000, 12, 3),
+    (1, 5, 1, 4800, 32, 4), (1, 5, 0, 16384, 32, 4)])
+def test_default_tilings(lib, pattern, radius, dtype, n, rows, wgs):
+    # sizes at which the rules of small, middle and large grids meet
+    t = Tuning()
+    check(lib, lib.prk_tuning_get(pattern, radius, dtype, n, C.byref(t)))
+    assert (t.rows_per_wave, t.wgs_per_cu) == (rows, wgs)
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 129, 513, 46340])
+def test_default_height_is_inside_the_grid(lib, n):
+    t = Tuning()
+    for pattern in (0, 1):
+        for radius in range(1, 9):
+            for dtype in (0, 1, 2):
+                check(lib, lib.prk_tuning_get(pattern, radius, dtype, n, C.byref(t)))
+                assert 1 <= t.rows_per_wave <= n
