@@ -63,7 +63,7 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 //  - An array of more than one and less than three (BF16: two) turns of two
 //    workgroups per CU takes the height that fills its turns best, the last
 //    one of which may be nearly empty, against the share of halo rows (FP64
-//    grid R=5, n = 4000: 24 rows 222 us, 32 rows 158; the FP32 grid R=5, four
+//    grid R=8, n = 2600: 24 rows 175 us, 32 rows 156; the FP32 grid R=5, four
 //    workgroups per CU, keeps its 32: n = 4800 76 us, 24 rows 90).  The
 //    middle's height stays unless another fills the turns clearly better, a
 //    lower one much better (FP64 star R=8, n = 2800: 24 rows 63.9 us, 12 rows,
