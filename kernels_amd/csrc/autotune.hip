@@ -47,7 +47,7 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 //    on (BF16 star R=8, n = 22000, half of the rows: 471 -> 414 us), the
 //    others lose (FP32 star R=5 641 -> 670), as do those of fewer points (BF16
 //    grid R=7, n = 18000, an eighth: 198 -> 236; not the FP64 star R=8, whose
-//    height is the same, n = 8504, an eighth: 69 -> 55).  Against the rule
+//    height is the same, n = 13000, a quarter: 307 -> 270).  Against the rule
 //    below for the middle: FP64 star R=8 1683 -> 1547 us; FP32 star R=5 797 ->
 //    730, grid R=5 1010 -> 901; BF16 star R=1 404 -> 380, grid R=6 942 -> 853.
 //    Stencils whose best at 16384 lost elsewhere keep the middle's (FP64 star
@@ -67,10 +67,11 @@ constexpr int kFinalists = 4;  // candidates timed again in the second stage
 //    workgroups per CU, keeps its 32: n = 4800 76 us, 24 rows 90).  The
 //    middle's height stays unless another fills the turns clearly better, a
 //    lower one much better (FP64 star R=8, n = 2800: 24 rows 63.9 us, 12 rows,
-//    by this measure 14 % better, 65.5), and where only a few workgroups lie
-//    past two turns (FP32: one), which cost nothing (FP32 grid R=6, n = 7000,
-//    half of the rows, 1029 workgroups of 24 rows: 111 us, one and a half
-//    turns of 32 rows 135).  Stars and grids of R <= 2 keep 8 rows.
+//    by this measure 14 % better, 65.5), and where what lies past the last
+//    whole turn is the last row of tiles alone, a short one: that costs
+//    nothing (FP32 grid R=6, n = 7000, half of the rows, 1029 workgroups of 24
+//    rows: 111 us, one and a half turns of 32 rows 135).  Stars and grids of R
+//    <= 2 keep 8 rows.
 //  - Where that is no more than one turn, the time is that of one wave going
 //    down its h + 2R rows, and lower tiles are faster until the chip is full:
 //    the lowest that give one workgroup per CU or two.  Two on a CU take 9/7
@@ -102,22 +103,22 @@ prk_tuning heuristic_tuning(int pattern, int radius, int dtype, int n, int nrows
     // 332 -> 349 us; 18000 485 -> 461), the wider ones gain from 12000 on.
     const int line = d == F64 ? 8000 : d == BF16 && R <= 3 ? 16000 : 12000;
     const bool arithmetic = p == 1 && ((d == F64 && R >= 3 && R <= 7) || (d == F32 && R == 5));
-    const bool wgs_alone = d == F64 && p == 0 && R == 8 && n >= line;  // the middle's height
+    const int lanes = d == F64 ? 128 : d == F32 ? 256 : 512;  // columns of a strip
+    constexpr long long kTurn = 512;  // workgroups
+    const long long groups = std::max(1, ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock);
+    auto tiles = [&](int h) { return groups * ((nrows + h - 1) / h); };
+    const bool wgs_alone = d == F64 && p == 0 && R == 8 && n >= line && tiles(rows) >= 3 * kTurn;  // the middle's height
     const bool large = wgs_alone || ((long long)n * nrows >= (long long)line * line && (nrows == n || R >= 6));
     if (large || arithmetic) {
         rows = kRows[d][p][R - 1];
         t.wgs_per_cu = kWgs[d][p][R - 1];
     }
-    const int lanes = d == F64 ? 128 : d == F32 ? 256 : 512;  // columns of a strip
-    constexpr long long kTurn = 512;  // workgroups
-    const long long groups = std::max(1, ((n + lanes - 1) / lanes + kWavesPerBlock - 1) / kWavesPerBlock);
-    auto tiles = [&](int h) { return groups * ((nrows + h - 1) / h); };
     // a second workgroup on a CU adds nothing to the FP64 grid R=8, and the
     // FP32 grid R=5 has four
     const long long lap = d == F64 && p == 1 && R == 8 ? kTurn / 2 : kTurn;
     const long long over = (tiles(rows) - 1) % lap + 1;  // workgroups of the last turn
-    const bool whole_turns = over <= 12 && (d == F32 || tiles(rows) > 2 * kTurn);
-    if ((R >= 3 || d == BF16) && tiles(rows) > kTurn && tiles(rows) < (d == BF16 ? 2 : 3) * kTurn && !whole_turns &&
+    const bool short_turn = over <= groups && 3 * ((nrows - 1) % rows + 1) <= 2 * rows;
+    if ((R >= 3 || d == BF16) && tiles(rows) > kTurn && tiles(rows) < (d == BF16 ? 2 : 3) * kTurn && !short_turn &&
         !(arithmetic && d == F32)) {
         static const int kHeights[] = {8, 12, 16, 24, 32};
         auto score = [&](int h) {  // share of its turns that the grid fills, times the share of rows that are no halo

@@ -772,18 +772,21 @@ __device__ inline void bstore_elem(__amdgpu_buffer_rsrc_t r, unsigned off, T v)
 //               Rows of 16 bytes or more: the vector must end in the next row.
 //   MODE_ELEM   element loads and stores (BF16 rows on odd elements, rows of
 //               under 16 bytes).
+//   MODE_LOADS  rows as in MODE_RAGGED: 16-byte loads, element stores
+//               (launch_pr takes it where it is the faster one).
 // Measured on MI355X, element accesses -> these: fused sweeps at n=9999, rows
 // on 128 bytes, FP32 star R=1 421 -> 274 us (n=10000: 274), FP64 star R=2
 // 640 -> 536, BF16 grid R=3 331 -> 167; at n=4001, pitch 4001, FP64 star R=2
 // 119 -> 96 us, FP32 71 -> 55.
-enum { MODE_ELEM = 0, MODE_VEC = 1, MODE_DWORD = 2, MODE_RAGGED = 3 };
+enum { MODE_ELEM = 0, MODE_VEC = 1, MODE_DWORD = 2, MODE_RAGGED = 3, MODE_LOADS = 4 };
+constexpr bool vec_stores(int mode) { return mode != MODE_ELEM && mode != MODE_LOADS; }
 
 // One row's V elements at byte offset off (kOOB: none).  `end`: the row is
 // the array's last (MODE_DWORD only).
 template <typename T, int V, int MODE, int AUX>
 __device__ inline u32x4 load_row_vec(__amdgpu_buffer_rsrc_t r, unsigned off, bool end)
 {
-    if (MODE == MODE_VEC || MODE == MODE_RAGGED || (MODE == MODE_DWORD && !end)) return bload16<AUX>(r, off);
+    if (MODE != MODE_ELEM && (MODE != MODE_DWORD || !end)) return bload16<AUX>(r, off);
     union { u32x4 v; T e[V]; } x;
 #pragma unroll
     for (int v = 0; v < V; ++v)
@@ -805,12 +808,12 @@ template <typename T, int V, int MODE, int AUX>
 __device__ inline void store_next_vec(__amdgpu_buffer_rsrc_t r, unsigned off, int cm, int n, bool ragged,
                                       const u32x4 &val)
 {
-    if (MODE == MODE_VEC || (MODE != MODE_ELEM && !ragged)) {
+    if (MODE == MODE_VEC || (vec_stores(MODE) && !ragged)) {
         bstore16<AUX>(r, off, val);
         return;
     }
-    const bool whole = MODE != MODE_ELEM && cm + V <= n;
-    if constexpr (MODE != MODE_ELEM) bstore16<AUX>(r, whole ? off : kOOB, val);
+    const bool whole = vec_stores(MODE) && cm + V <= n;
+    if constexpr (vec_stores(MODE)) bstore16<AUX>(r, whole ? off : kOOB, val);
     union { u32x4 v; T e[V]; } x;
     x.v = val;
 #pragma unroll
@@ -955,7 +958,7 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = FRAME == FRAME_KEEP && MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = FRAME == FRAME_KEEP && vec_stores(MODE) && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1043,13 +1046,13 @@ __device__ inline void wave_tile_impl(const void *in_, void *in_next_, void *out
                 union { u32x4 v; T e[V]; } res;
                 compute_points<DT, P, R, V, HP>(rows, cur.outv.e, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE != MODE_ELEM && FRAME == FRAME_REWRITE) {
+                if constexpr (vec_stores(MODE) && FRAME == FRAME_REWRITE) {
                     unsigned off[V];
                     out_offsets<V, ES>(c0, n, R, off);
 #pragma unroll
                     for (int v = 0; v < V; ++v) res.e[v] = off[v] != kOOB ? res.e[v] : cur.outv.e[v];
                     bstore16<AUX_STREAM>(rout, off_main, res.v);
-                } else if constexpr (MODE != MODE_ELEM) {
+                } else if constexpr (vec_stores(MODE)) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {
@@ -1106,7 +1109,7 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = vec_stores(MODE) && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1190,7 +1193,7 @@ __device__ inline void wave_tile_star(const void *in_, void *in_next_, void *out
                 Vec res;
                 star_points<DT, R, V, HP>(&ring[cs][HP + lane * V], col, sd.outv.e, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE != MODE_ELEM) {
+                if constexpr (vec_stores(MODE)) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {
@@ -1232,7 +1235,7 @@ __device__ inline void wave_tile_grid2(const void *in_, void *in_next_, void *ou
 
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
-    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = vec_stores(MODE) && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1322,7 +1325,7 @@ __device__ inline void wave_tile_grid2(const void *in_, void *in_next_, void *ou
 #pragma unroll
                     for (int v = 0; v < V; ++v) res.e[v] = cur[m].outv.e[v] + sum[m][v];
                     const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)(o + m) * pitch, st_bytes);
-                    if constexpr (MODE != MODE_ELEM) {
+                    if constexpr (vec_stores(MODE)) {
                         if (!edge) {
                             bstore16<AUX_STREAM>(rout, off_main, res.v);
                         } else {
@@ -1486,7 +1489,7 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
     const int lo = max(r0 - R, 0), hi = min(r1 + R, sp.nrows);
     const int olo = max(r0, R), ohi = min(r1, sp.nrows - R);
     // edge waves park their straddling vectors (tiles of at most kStashRows output rows)
-    u32x4 *const stash = MODE != MODE_ELEM && ohi - olo <= kStashRows ? stash_lds : nullptr;
+    u32x4 *const stash = vec_stores(MODE) && ohi - olo <= kStashRows ? stash_lds : nullptr;
     const int ulo = max(r0, sp.upd_lo), uhi = min(r1, sp.upd_hi);
 
     const T *in = (const T *)in_;
@@ -1559,7 +1562,7 @@ __device__ inline void wave_tile_rw(const void *in_, void *in_next_, void *out_,
                 union { u32x4 v; T e[V]; } res;
                 from_f32_vec<V>(f, res.e);
                 const __amdgpu_buffer_rsrc_t rout = row_rsrc(out + (long long)o * pitch, st_bytes);
-                if constexpr (MODE != MODE_ELEM) {
+                if constexpr (vec_stores(MODE)) {
                     if (!edge) {
                         bstore16<AUX_STREAM>(rout, off_main, res.v);
                     } else {

@@ -56,7 +56,7 @@ int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hip
     // kStashRows rows of out from one resource, which must stay below the
     // out-of-range offset.
     a.stash = 0;
-    if (!RW && MODE != MODE_ELEM &&
+    if (!RW && vec_stores(MODE) &&
         (long long)kStashRows * p.pitch * (long long)sizeof(typename G::T) < (long long)kOOB) {
         if (dyn >= kStashBytes) {
             a.stash = 1;
@@ -78,10 +78,10 @@ int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hip
 
 // The fused sweep of aligned rows is the hot path: it is instantiated for
 // every pipeline depth / cache policy the tuner chooses from (radii beyond
-// the reference's 5: one, two rows in flight with non-temporal stores).  The
-// other forms have one variant each.  Four rows in flight (variant 8) made FP64
-// star R=2 at n=30000 1.3-1.8 % faster than three at 6- and 8-row blocks
-// on MI355X (alternating runs on one box), and slower at 12 and 16 rows.
+// the reference's 5: one, two rows in flight with non-temporal stores).  Four
+// rows in flight (variant 8) made FP64 star R=2 at n=30000 1.3-1.8 % faster
+// than three at 6- and 8-row blocks on MI355X (alternating runs on one box),
+// and slower at 12 and 16 rows.
 template <int DT, int P, int R>
 int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipStream_t s)
 {
@@ -107,19 +107,50 @@ int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipS
             }
         }
     }
-    // Rows in flight and non-temporal out of the other forms: the default of
-    // the fused sweep (unfused FP64 star R=2, two rows and temporal before:
-    // n = 16384 1146 -> 1071 us, pitch 4001 92 -> 82).
+    // The other forms: arrays past the last-level cache, or in the L2s
+    // together, with the rows in flight and the non-temporal stores of the
+    // default fused sweep, arrays between (`cached`) with their stores through
+    // the cache.  Measured on MI355X, FP64 star R=2 unless said otherwise:
+    //  - unfused, then in += 1: n = 16384 1146 us temporal, 1071 non-temporal;
+    //    n = 1500 22.3, 25.6; n = 700 10.1, 9.4.
+    //  - fused, ragged rows: FP64 inside the last-level cache takes element
+    //    stores (n = 2301 31.0 us, vectors 32.3, non-temporal ones 33.3; n =
+    //    4001 102, 91.8, 85.9), FP32 grid R=4 vectors (n = 4001 50.2,
+    //    non-temporal 60.7, element stores 49.1; star R=4, n = 1801 14.2, 15.3,
+    //    15.7), so does BF16 (stencils' mean at 4001 7 % over non-temporal).
+    //    The widest grids are bound by their arithmetic, and the vectors'
+    //    registers cost more than their stores save (FP64 grid R=8, n = 6501
+    //    809 us, vectors 849; FP32 grid R=8, n = 8001 402, 444).
+    //  - fused, rows off 16 bytes: FP64 inside the last-level cache by element
+    //    (n = 3101 56.4 us, vectors 57.9, non-temporal 62.3).
     constexpr int PF = R > kRefMaxRadius ? 2 : 3;
+    const long long bytes = (fuse ? 3 : 2) * (long long)p.span.nrows * p.pitch * (long long)sizeof(typename SweepGeom<DT, R>::T);
+    const bool fits = bytes <= kLastLevelCache, cached = fits && bytes > kInL2;
     if (fuse) {
-        if (p.mode == MODE_RAGGED) return launch_one<DT, P, R, true, MODE_RAGGED, PF, 1>(p, in, in_next, out, s);
-        if (p.mode == MODE_DWORD) return launch_one<DT, P, R, true, MODE_DWORD, PF, 1>(p, in, in_next, out, s);
+        if (p.mode == MODE_RAGGED) {
+            constexpr bool wide = P == GRID && R >= (DT == F64 ? 8 : DT == F32 ? 6 : kMaxRadius + 1);
+            if constexpr (DT == F64) {
+                if (wide || fits) return launch_one<DT, P, R, true, MODE_LOADS, kPrefetch, 0>(p, in, in_next, out, s);
+            } else if constexpr (wide) {
+                return launch_one<DT, P, R, true, MODE_LOADS, kPrefetch, 0>(p, in, in_next, out, s);
+            } else {
+                if (cached) return launch_one<DT, P, R, true, MODE_RAGGED, PF, 0>(p, in, in_next, out, s);
+            }
+            if constexpr (!wide) return launch_one<DT, P, R, true, MODE_RAGGED, PF, 1>(p, in, in_next, out, s);
+        }
+        if (p.mode == MODE_DWORD && !(DT == F64 && fits))
+            return launch_one<DT, P, R, true, MODE_DWORD, PF, 1>(p, in, in_next, out, s);
         return launch_one<DT, P, R, true, MODE_ELEM, kPrefetch, 0>(p, in, in_next, out, s);
+    }
+    if (p.mode == MODE_ELEM) return launch_one<DT, P, R, false, MODE_ELEM, kPrefetch, 0>(p, in, in_next, out, s);
+    if (cached) {
+        if (p.mode == MODE_VEC) return launch_one<DT, P, R, false, MODE_VEC, kPrefetch, 0>(p, in, in_next, out, s);
+        if (p.mode == MODE_RAGGED) return launch_one<DT, P, R, false, MODE_RAGGED, kPrefetch, 0>(p, in, in_next, out, s);
+        return launch_one<DT, P, R, false, MODE_DWORD, kPrefetch, 0>(p, in, in_next, out, s);
     }
     if (p.mode == MODE_VEC) return launch_one<DT, P, R, false, MODE_VEC, PF, 1>(p, in, in_next, out, s);
     if (p.mode == MODE_RAGGED) return launch_one<DT, P, R, false, MODE_RAGGED, PF, 1>(p, in, in_next, out, s);
-    if (p.mode == MODE_DWORD) return launch_one<DT, P, R, false, MODE_DWORD, PF, 1>(p, in, in_next, out, s);
-    return launch_one<DT, P, R, false, MODE_ELEM, kPrefetch, 0>(p, in, in_next, out, s);
+    return launch_one<DT, P, R, false, MODE_DWORD, PF, 1>(p, in, in_next, out, s);
 }
 
 template <int DT>
