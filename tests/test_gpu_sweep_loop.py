@@ -70,3 +70,53 @@ def test_refresh_by_size(gpu, n):
     want = t + 1.0
     K.add(n, 32, t)
     assert torch.equal(t, want)
+
+
+@pytest.mark.parametrize("dtype", [F64, F32, BF16])
+@pytest.mark.parametrize("pattern,radius", [(p, r) for p in (0, 1) for r in range(1, 9)])
+def test_sweep_by_sweep_bitwise(gpu, oracle, pattern, radius, dtype):
+    # whole vectors, ragged rows, and rows off 16 bytes, default tiling
+    strip, sweeps = 64 * (2, 4, 8)[dtype], 5
+    for n, pitch in ((2 * radius + 1, None), (strip, None), (strip + 1, None), (131 + radius, 131 + radius)):
+        print(f"sweeps p{pattern} r{radius} d{dtype} n={n} pitch={pitch}", flush=True)
+        bufs = [K.alloc_grid(n, dtype, pitch=pitch) for _ in range(3)]
+        K.init(K.INIT_SEEDED, 31 + n, dtype, bufs[0], bufs[2])
+        fin = loop(pattern, radius, dtype, bufs, sweeps)
+        if dtype == F64:
+            ref_out, ref_in = oracle.run(pattern, radius, n, 32, sweeps - 1, 1, 31 + n)
+        else:
+            ref_out, ref_in = oracle.run_lp(dtype, pattern, radius, n, sweeps - 1, 1, 31 + n)
+        assert np.array_equal(bits(host(bufs[2])), bits(ref_out)), (n, pitch)
+        assert np.array_equal(bits(host(fin)), bits(ref_in)), (n, pitch)
+
+
+@pytest.mark.parametrize("dtype,pattern,radius", [(F64, 0, 4), (F64, 1, 3), (F32, 0, 4), (F32, 1, 2), (BF16, 0, 7)])
+def test_sweeps_of_the_tuned_tiling(gpu, oracle, dtype, pattern, radius):
+    # the tiling that the search recorded, without an override
+    n, sweeps = 256, 3
+    bufs = [K.alloc_grid(n, dtype) for _ in range(3)]
+    try:
+        tuned, got = K.autotune(pattern, radius, dtype, *bufs, reps=1), K.Tuning()
+        K.check(K.lib().prk_tuning_get(pattern, radius, dtype, n, got))
+        assert (got.variant, got.rows_per_wave) == (tuned.variant, tuned.rows_per_wave)
+        K.init(K.INIT_SEEDED, 4, dtype, bufs[0], bufs[2])
+        loop(pattern, radius, dtype, bufs, sweeps)
+        assert np.array_equal(bits(host(bufs[2])), bits(band(oracle, dtype, pattern, radius, n, sweeps - 1, 4, 0, n)))
+    finally:
+        K.check(K.lib().prk_tuning_clear())
+
+
+@pytest.mark.parametrize("dtype,n,pattern,radius", [(F64, 30000, 0, 2), (F64, 30000, 1, 2), (F64, 16384, 1, 5),
+                                                    (F32, 30000, 0, 2), (BF16, 30000, 1, 3)])
+def test_large_grid_sweeps_on_bands(gpu, oracle, dtype, n, pattern, radius):
+    bufs, sweeps = [K.alloc_grid(n, dtype) for _ in range(3)], 2
+    K.init(K.INIT_SEEDED, 42, dtype, bufs[0], bufs[2])
+    loop(pattern, radius, dtype, bufs, sweeps)
+    rng = np.random.default_rng(7)
+    spans = [(0, radius + 4), (n - radius - 4, n)] + [(int(a), int(a) + 8) for a in rng.integers(0, n - 8, 6)]
+    for rows in (8, 12, 32):  # across tile boundaries in the middle
+        c = n // 2 // rows * rows
+        spans.append((c - 3, c + 3))
+    for a, b in spans:
+        ref = band(oracle, dtype, pattern, radius, n, sweeps - 1, 42, a, b)
+        assert np.array_equal(bits(host(bufs[2][a:b])), bits(ref)), (a, b)
