@@ -7,10 +7,11 @@
 // writes A + 1 back to the same addresses, and parks the tile in LDS (rows
 // padded by one element so that reading a column spreads over the banks).
 // Then it issues the loads of the matching rows of B, waits for the others'
-// share of the tile, adds the tile's columns to B and stores it.  Every element of A and B is read once
-// and written once: 32 bytes per element, the algorithmic traffic of the
-// reference's Rate (4 * 8 * order^2 bytes).  What bounds it is HBM, at the
-// rate the tiles' short row segments reach (launch_transpose).
+// share of the tile, adds the tile's columns to B and stores it.  Every element
+// of A and B is read once and written once: 32 bytes per element, the
+// algorithmic traffic of the reference's Rate (4 * 8 * order^2 bytes).  What
+// bounds it is HBM, at the rate the tiles' short row segments reach
+// (launch_transpose).
 // Edges: rows and columns beyond `order` are out-of-range buffer offsets
 // (reads give 0, writes are dropped).  Where order is odd, rows start on
 // 8-byte boundaries, which the 16-byte accesses take as they are; the tiles
@@ -87,15 +88,17 @@ __device__ inline void store2(__amdgpu_buffer_rsrc_t r, unsigned off, bool last,
     }
 }
 
-// One TR x TC tile of A (TR rows, TC columns) on NTH threads.  NT: loads and
-// stores marked non-temporal.
-template <int TR, int TC, int NTH, bool NT, bool SPLIT>
+// Non-temporal accesses of a tile.
+enum { NT_NONE = 0, NT_STORES = 1, NT_ALL = 3 };
+
+// One TR x TC tile of A (TR rows, TC columns) on NTH threads.
+template <int TR, int TC, int NTH, int NT, bool SPLIT>
 __device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, double (*tile)[TC + 1])
 {
     constexpr int LPR1 = TC / 2, RPP1 = NTH / LPR1, NP1 = TR / RPP1;  // A rows
     constexpr int LPR2 = TR / 2, RPP2 = NTH / LPR2, NP2 = TC / RPP2;  // B rows
     static_assert(NP1 >= 1 && NP2 >= 1 && RPP1 * NP1 == TR && RPP2 * NP2 == TC, "tile shape");
-    constexpr int AUX = NT ? 2 : 0;
+    constexpr int AUX_LD = NT & 2 ? 2 : 0, AUX_ST = NT & 1 ? 2 : 0;
     const int order = a.order;
     const unsigned row_bytes = (unsigned)order * 8u;
     union V { u32x4 v; double d[2]; };
@@ -118,7 +121,7 @@ __device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, do
 
     V x[NP1], y[NP2];
 #pragma unroll
-    for (int p = 0; p < NP1; ++p) x[p].v = load2<AUX, SPLIT>(ra, off_a + p * step_a, last_a);
+    for (int p = 0; p < NP1; ++p) x[p].v = load2<AUX_LD, SPLIT>(ra, off_a + p * step_a, last_a);
 #pragma unroll
     for (int p = 0; p < NP1; ++p) {
         V z;
@@ -126,22 +129,22 @@ __device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, do
         z.d[1] = x[p].d[1] + 1.0;
         tile[p * RPP1 + ar][ac] = x[p].d[0];
         tile[p * RPP1 + ar][ac + 1] = x[p].d[1];
-        store2<AUX, SPLIT>(ra, off_a + p * step_a, last_a, z.v);
+        store2<AUX_ST, SPLIT>(ra, off_a + p * step_a, last_a, z.v);
     }
 #pragma unroll
-    for (int p = 0; p < NP2; ++p) y[p].v = load2<AUX, SPLIT>(rb, off_b + p * step_b, last_b);
+    for (int p = 0; p < NP2; ++p) y[p].v = load2<AUX_LD, SPLIT>(rb, off_b + p * step_b, last_b);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p < NP2; ++p) {
         y[p].d[0] = y[p].d[0] + tile[bc][p * RPP2 + br];
         y[p].d[1] = y[p].d[1] + tile[bc + 1][p * RPP2 + br];
-        store2<AUX, SPLIT>(rb, off_b + p * step_b, last_b, y[p].v);
+        store2<AUX_ST, SPLIT>(rb, off_b + p * step_b, last_b, y[p].v);
     }
 }
 
 // ODD: order is odd; the tiles that hold the last column of A or B split
 // their vectors.
-template <int TR, int TC, int NTH, bool NT, bool ODD>
+template <int TR, int TC, int NTH, int NT, bool ODD>
 __global__ __launch_bounds__(NTH) void transpose_kernel(TransposeArgs a)
 {
     __shared__ double tile[TR][TC + 1];
@@ -153,7 +156,9 @@ __global__ __launch_bounds__(NTH) void transpose_kernel(TransposeArgs a)
         transpose_tile<TR, TC, NTH, NT, false>(a, tr, tc, tile);
 }
 
-// One 64 x 64 tile of A in 8-byte accesses, non-temporal stores.
+// One 64 x 64 tile of A in 8-byte accesses, non-temporal stores, a resource
+// for each row (one for the tile took 1 to 5 % longer above order 13000: 18473
+// 2341 us, 2390; 14497 1632, 1715).
 __global__ __launch_bounds__(256) void transpose_kernel_8b(TransposeArgs a)
 {
     constexpr int T = 64, RPP = 4, NP = T / RPP;  // four rows at a time
@@ -162,27 +167,30 @@ __global__ __launch_bounds__(256) void transpose_kernel_8b(TransposeArgs a)
     tile_of_transpose(a, blockIdx.x, tr, tc);
     const int order = a.order;
     const unsigned row_bytes = (unsigned)order * 8u;
-    const __amdgpu_buffer_rsrc_t ra =
-        row_rsrc(a.A + (long long)tr * T * order, (unsigned)min(T, order - tr * T) * row_bytes);
-    const __amdgpu_buffer_rsrc_t rb =
-        row_rsrc(a.B + (long long)tc * T * order, (unsigned)min(T, order - tc * T) * row_bytes);
-    const int r = threadIdx.x / T, c = threadIdx.x % T;
-    const unsigned step = RPP * row_bytes;
-    const unsigned off_a = tc * T + c < order ? r * row_bytes + (unsigned)(tc * T + c) * 8u : kOOB;
-    const unsigned off_b = tr * T + c < order ? r * row_bytes + (unsigned)(tr * T + c) * 8u : kOOB;
+    const int r = threadIdx.x / T, c = threadIdx.x - r * T;
+    const unsigned off_a = tc * T + c < order ? (unsigned)(tc * T + c) * 8u : kOOB;
+    const unsigned off_b = tr * T + c < order ? (unsigned)(tr * T + c) * 8u : kOOB;
+    __amdgpu_buffer_rsrc_t rs[NP];
     double x[NP];
+    auto load = [&](const double *m, int row0, unsigned off) {
 #pragma unroll
-    for (int p = 0; p < NP; ++p) x[p] = bload_elem<double, 0>(ra, off_a + p * step);
+        for (int p = 0; p < NP; ++p) {
+            const int row = row0 + p * RPP + r;
+            const bool ok = row < order;
+            rs[p] = row_rsrc(m + (long long)(ok ? row : 0) * order, ok ? row_bytes : 0u);
+            x[p] = bload_elem<double, 0>(rs[p], off);
+        }
+    };
+    load(a.A, tr * T, off_a);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         tile[p * RPP + r][c] = x[p];
-        bstore_elem<double, 2>(ra, off_a + p * step, x[p] + 1.0);
+        bstore_elem<double, 2>(rs[p], off_a, x[p] + 1.0);
     }
     __syncthreads();
+    load(a.B, tc * T, off_b);
 #pragma unroll
-    for (int p = 0; p < NP; ++p) x[p] = bload_elem<double, 0>(rb, off_b + p * step);
-#pragma unroll
-    for (int p = 0; p < NP; ++p) bstore_elem<double, 2>(rb, off_b + p * step, x[p] + tile[c][p * RPP + r]);
+    for (int p = 0; p < NP; ++p) bstore_elem<double, 2>(rs[p], off_b, x[p] + tile[c][p * RPP + r]);
 }
 
 // One 128 x 128 tile of A on 1024 threads, in two halves through 66 KiB of
@@ -348,21 +356,23 @@ int transpose_args(int order, const double *A, const double *B)
 int g_tr_shape = -1, g_tr_mode = -1;  // -1: the defaults below
 
 template <int TR, int TC, int NTH = 256>
-int launch_shape(TransposeArgs a, bool large, hipStream_t s)
+int launch_shape(TransposeArgs a, int nt, hipStream_t s)
 {
     a.ntr = (a.order + TR - 1) / TR;
     a.ntc = (a.order + TC - 1) / TC;
     const unsigned blocks = (unsigned)a.ntr * (unsigned)a.ntc;
-    // large: one workgroup per CU of the 64 x 128 tiles (more than half of
+    // NT_ALL: one workgroup per CU of the 64 x 128 tiles (more than half of
     // its LDS each)
     constexpr size_t lds = sizeof(double) * TR * (TC + 1), half = 80u * 1024u;
-    const size_t dyn = large && lds > half / 2 && lds < half ? half + 4096u - lds : 0;
+    const size_t dyn = nt == NT_ALL && lds > half / 2 && lds < half ? half + 4096u - lds : 0;
     if (a.order & 1)
-        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, false, true>), dim3(blocks), dim3(NTH), 0, s, a);
-    else if (large)
-        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, true, false>), dim3(blocks), dim3(NTH), dyn, s, a);
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_NONE, true>), dim3(blocks), dim3(NTH), 0, s, a);
+    else if (nt == NT_ALL)
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_ALL, false>), dim3(blocks), dim3(NTH), dyn, s, a);
+    else if (nt == NT_STORES)
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_STORES, false>), dim3(blocks), dim3(NTH), 0, s, a);
     else
-        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, false, false>), dim3(blocks), dim3(NTH), 0, s, a);
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_NONE, false>), dim3(blocks), dim3(NTH), 0, s, a);
     return check_hip(hipGetLastError(), "transpose launch");
 }
 
@@ -391,39 +401,36 @@ int launch_2h(TransposeArgs a, hipStream_t s)
 //  - Up to 4096 64 x 128 tiles, loads and stores through the caches: both
 //    matrices stay in the 256 MB of the last one (order 2000: 19; 4096: 79,
 //    93 non-temporal; 64 x 64 tiles in 8-byte accesses at 3001: 56, these 48).
-//  - Above, rows on 64-byte boundaries: the same tiles, everything
-//    non-temporal and one workgroup at a time on a CU: order 32768 6005 (two
-//    workgroups 6150, only the stores non-temporal 6540), 16384 1490 (1520,
-//    1630), 9000 529 (533, 598), 20004 3071 (3106, 3379).
-//  - Rows off them share cache lines between tiles, and what one tile leaves
-//    of a line must wait in the cache for the next: 32 x 32 tiles without
-//    hints (order 10002 685, the tiles above 817 and with only the stores
-//    non-temporal 787; 16380 1744, 2098, 2043).  From 20004 on rows on
-//    32-byte boundaries do better with the tiles above (30004: 6975 against
-//    7837).
+//  - Above, the same tiles, and only the stores non-temporal.  Rows on 64-byte
+//    boundaries share no cache line between tiles, so from 4800 on their loads
+//    are non-temporal too, with one workgroup at a time on a CU: order 32768
+//    6005 (two workgroups 6150, only the stores non-temporal 6540), 16384 1490
+//    (1520, 1630), 9000 529 (533, 598), 4808 150 (151 the stores alone; 4504
+//    112, 107).  Other rows lose by non-temporal loads (10002 817, 787).  32 x
+//    32 tiles without hints take them in between, but by where the rows fall on
+//    the memory's channels: 18 % faster at 21050, 18 % slower at 24006.
 //  - Odd orders and matrices off 16-byte boundaries: 64 x 64 tiles in 8-byte
-//    accesses (order 12289 1091, 32 x 32 tiles 1192, 64 x 128 1251).
+//    accesses (order 12289 1091, 64 x 128 1251).
 int launch_transpose(int order, double *A, double *B, hipStream_t s)
 {
     TransposeArgs a{A, B, order, 0, 0, g_tr_mode < 0 ? 0 : g_tr_mode};
-    const bool aligned = order % 2 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
-    const bool large = order > 4096;
-    if (large && !aligned) return launch_8b(a, s);
-    if (large && g_tr_shape < 0 && (order % 4 != 0 || (order % 8 != 0 && order <= 16384)))
-        return launch_shape<32, 32>(a, false, s);
+    const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B;
+    const bool aligned = order % 2 == 0 && ptrs % 16 == 0;
+    if (order > 4096 && !aligned) return launch_8b(a, s);
+    const int nt = order <= 4096 ? NT_NONE : order >= 4800 && order % 8 == 0 && ptrs % 64 == 0 ? NT_ALL : NT_STORES;
     const int shape = order <= 1024 ? 3 : 2;
     switch (g_tr_shape < 0 ? shape : g_tr_shape) {
-    case 1: return launch_shape<128, 64>(a, large, s);
-    case 2: return launch_shape<64, 128>(a, large, s);
-    case 3: return launch_shape<32, 64>(a, large, s);
-    case 4: return launch_shape<128, 128, 1024>(a, large, s);
-    case 5: return launch_shape<32, 256>(a, large, s);
-    case 6: return launch_shape<256, 32>(a, large, s);
-    case 7: return launch_shape<64, 128, 512>(a, large, s);
+    case 1: return launch_shape<128, 64>(a, nt, s);
+    case 2: return launch_shape<64, 128>(a, nt, s);
+    case 3: return launch_shape<32, 64>(a, nt, s);
+    case 4: return launch_shape<128, 128, 1024>(a, nt, s);
+    case 5: return launch_shape<32, 256>(a, nt, s);
+    case 6: return launch_shape<256, 32>(a, nt, s);
+    case 7: return launch_shape<64, 128, 512>(a, nt, s);
     case 8:
         if (aligned) return launch_2h(a, s);
-        return launch_shape<64, 64>(a, large, s);
-    default: return launch_shape<64, 64>(a, large, s);
+        return launch_shape<64, 64>(a, nt, s);
+    default: return launch_shape<64, 64>(a, nt, s);
     }
 }
 
