@@ -93,3 +93,29 @@ def test_server_host_logic(tmp_path, sanitizer, args, gbs):
     assert updates > 0
     assert "WARNING: ThreadSanitizer" not in r.stderr and "ERROR: AddressSanitizer" not in r.stderr
     assert "runtime error" not in r.stderr
+
+
+def test_windows_hold_eight_stages_without_passes(tmp_path):
+    """A request whose stencil has no pass kernel advances one sweep a stage:
+    its 50 iterations (54 stages) are answered in 7 windows; with passes of 6
+    sweeps two stages a window are enough (init, 9 passes, norm: 6 windows)."""
+    objs = []
+    for src in SOURCES[:2]:
+        obj = tmp_path / (src.name + ".o")
+        subprocess.run([HIPCC, "--offload-host-only", "-O1", "-std=c++17", "-fPIC", f"-I{ROOT / 'include'}",
+                        f"-I{ROOT / 'kernels_amd/csrc'}", "-x", "hip", "-c", str(src), "-o", str(obj)],
+                       check=True, capture_output=True, text=True)
+        objs.append(str(obj))
+    so = tmp_path / "libserver.so"
+    subprocess.run([CLANG, "-shared", "-Wl,-Bsymbolic", "-o", str(so), *objs, "-lpthread"], check=True,
+                   capture_output=True, text=True)
+    code = ("from kernels_amd.server import Server\n"
+            "for spec in ((1, 3, 2, 64, 50, 1, 1), (0, 2, 1, 64, 50, 1, 1)):\n"
+            "    s = Server(budget_bytes=1 << 30)\n"
+            "    s.submit(spec)\n"
+            "    s.drain(60)\n"
+            "    print(s.stats()['windows'], s.poll()[0]['norm'])\n"
+            "    s.close()\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, cwd=ROOT,
+                       env=dict(os.environ, PRK_STENCIL_LIB=str(so)))
+    assert r.stdout.split() == ["7", "102.0", "6", "102.0"], r.stdout + r.stderr[-2000:]
