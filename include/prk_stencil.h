@@ -284,9 +284,11 @@ void prk_batch_destroy(prk_batch *b);
  * times each candidate height (16, 32, 64, 128 rows) over `reps` graph
  * replays of a batch of that group alone (repeated until its rounds fill
  * the GPU), and records the fastest if it beats the default 32 rows by at
- * least 5 %; it blocks, and writes the number of keys tuned.  prk_batch_create with
- * rows_per_tile = 0 then takes each grid's height from the table (32 rows
- * for keys not tuned).  Heights never change results.
+ * least 5 %; it blocks, and writes the number of keys tuned.  Keys whose
+ * stencil runs in passes have no height to tune: they are counted, and nothing
+ * is timed or recorded.  prk_batch_create with rows_per_tile = 0 then takes
+ * each grid's height from the table (32 rows for keys not tuned).  Heights
+ * never change results.
  * prk_batch_tuning_get reports the height a grid would get. */
 int prk_batch_autotune(const prk_solve *solves, int count, int sample, int reps, int *keys_tuned);
 int prk_batch_tuning_get(int pattern, int radius, int dtype, int n, int *rows);

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <tuple>
 #include <vector>
 
@@ -446,7 +447,10 @@ int prk_batch_create(const prk_solve *solves, int count, int rows_per_tile, int 
     for (int i = 0; i < count; ++i) {
         const int c = batch_class_of(solves[i]);
         ids[c].push_back(i);
-        const long long w = (long long)(solves[i].iterations + 1) * b->grids[i].ntiles;
+        // (of passes by tiles of the default height: a recorded height is not theirs)
+        const BGrid &g = b->grids[i];
+        const int h = batch_has_passes(g) ? std::min(g.n, default_tile_rows(g.radius)) : g.rows;
+        const long long w = (long long)(solves[i].iterations + 1) * g.strips * ((g.n + h - 1) / h);
         cwork[c] += w;
         all_work += w;
     }
@@ -678,8 +682,15 @@ int prk_batch_autotune(const prk_solve *solves, int count, int sample, int reps,
     int rc;
     for (int i = 0; i < count; ++i)
         if ((rc = validate_solve(solves[i]))) return rc;
+    // Passes have tiles of kBatchPassRows whatever the table holds: their keys
+    // count as tuned, with nothing timed or recorded.
     std::map<BKey, std::vector<prk_solve>> picked;
+    std::set<BKey> passes;
     for (int i = 0; i < count; ++i) {
+        if (pass_built(solves[i].pattern, solves[i].radius, solves[i].dtype)) {
+            passes.insert(batch_key(solves[i]));
+            continue;
+        }
         std::vector<prk_solve> &g = picked[batch_key(solves[i])];
         if ((int)g.size() < sample) {
             prk_solve t = solves[i];
@@ -707,7 +718,7 @@ int prk_batch_autotune(const prk_solve *solves, int count, int sample, int reps,
     rc = check_hip(hipStreamCreateWithFlags(&st, hipStreamNonBlocking), "autotune stream");
     if (!rc) rc = check_hip(hipEventCreate(&e0), "event");
     if (!rc) rc = check_hip(hipEventCreate(&e1), "event");
-    int tuned = 0;
+    int tuned = (int)passes.size();
     for (auto &kv : groups) {
         if (rc) break;
         const std::vector<prk_solve> &sub = kv.second;

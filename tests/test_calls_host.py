@@ -163,3 +163,30 @@ def test_default_height_is_inside_the_grid(lib, n):
             for dtype in (0, 1, 2):
                 check(lib, lib.prk_tuning_get(pattern, radius, dtype, n, C.byref(t)))
                 assert 1 <= t.rows_per_wave <= n
+
+
+def test_batch_heights_of_passes_are_not_tuned(lib):
+    # a stencil that runs in passes ignores the table of heights: nothing is
+    # timed for it, and what the table holds leaves the schedule as it is
+    L, keys, rows = lib, C.c_int(), C.c_int()
+    solves = (Solve * 6)(*[Solve(0, 2, 1, 300 + k, 9, 1, k) for k in range(3)],
+                         *[Solve(1, 6, 1, 300 + k, 9, 1, k) for k in range(3)])
+
+    def plan():
+        batch, info = C.c_void_p(), (C.c_longlong(), C.c_longlong(), C.c_int())
+        check(L, L.prk_batch_create(solves, 6, 0, 0, C.byref(batch)))
+        check(L, L.prk_batch_info(batch, *[C.byref(v) for v in info]))
+        L.prk_batch_destroy(batch)
+        return [v.value for v in info]
+
+    try:
+        before = plan()
+        L.mock_reset()
+        check(L, L.prk_batch_autotune(solves, 3, 2, 1, C.byref(keys)))
+        assert keys.value == 1 and L.mock_kernels() == 0
+        check(L, L.prk_batch_tuning_set(0, 2, 1, 300, 128))
+        assert plan()[1:] == before[1:]
+        check(L, L.prk_batch_autotune(solves, 6, 2, 1, C.byref(keys)))
+        assert keys.value == 2 and L.mock_kernels() > 0
+    finally:
+        L.prk_batch_tuning_clear()
