@@ -164,7 +164,7 @@ int prk_l1norm_noalloc(int dtype, int n, long long pitch, int radius, const void
  * timed sweeps 1..iterations, unless it is part of the one pass that an even
  * number of iterations then takes.  *final_in_buf receives 0 or 1 (the buffer
  * holding in after the last refresh; iterations + 1 odd: 1), the other buffer
- * holds an earlier in.  *avg_seconds: the mean time of one timed sweep, where
+ * holds the in before it.  *avg_seconds: the mean time of one timed sweep, where
  * sweep 0 is in the pass that of all iterations + 1.  Synchronous. */
 int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iterations,
             void *buf0, void *buf1, void *out, void *stream, int *final_in_buf,
