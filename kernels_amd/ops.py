@@ -40,10 +40,10 @@ def _good_grids(dtype: int, grids: tuple, square: bool, rows: int | None) -> tup
     """The (rows, pitch) of _check_grids where everything holds that it
     checks, in one pass over the grids; None where something may not."""
     want, ref = _TORCH.get(dtype), grids[0] if grids else None
-    if want is None or not isinstance(ref, torch.Tensor):
+    if want is None or not isinstance(ref, torch.Tensor) or ref.dtype is not want or ref.dim() != 2:
         return None
     shape, stride, device = ref.shape, ref.stride(), ref.get_device()
-    if len(shape) != 2 or stride[1] != 1 or device < 0:
+    if stride[1] != 1 or device < 0:
         return None
     nrows, ncols = shape
     pitch = stride[0] if nrows > 1 else max(stride[0], ncols)

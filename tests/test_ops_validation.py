@@ -90,3 +90,12 @@ def test_default_pitch():
             assert p >= n and (p * es) % align == 0 and (p - n) * es < align, (dtype, n, p)
     assert K.default_pitch(30000, K.F64) == 30080 and K.default_pitch(30000, K.BF16) == 30016
     assert K.default_pitch(16384, K.F32) == 16384
+
+
+def test_tensors_without_strides_are_refused_by_type_and_shape_first():
+    with pytest.raises(ValueError, match="storage type"):
+        _check_grids(K.F64, torch.zeros((4, 4), dtype=torch.float32).to_sparse())
+    with pytest.raises(ValueError, match="storage type"):
+        _check_grids(K.F64, grid(4), torch.zeros((4, 4), dtype=torch.float32).to_sparse())
+    with pytest.raises(ValueError, match="unit column stride"):
+        _check_grids(K.F64, torch.zeros(8, dtype=torch.float64))
