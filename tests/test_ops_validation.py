@@ -94,8 +94,8 @@ def test_default_pitch():
 
 def test_tensors_without_strides_are_refused_by_type_and_shape_first():
     with pytest.raises(ValueError, match="storage type"):
-        _check_grids(K.F64, torch.zeros((4, 4), dtype=torch.float32).to_sparse())
+        _check_grids(K.F64, torch.zeros((4, 4), dtype=torch.float32).to_sparse_csr())
     with pytest.raises(ValueError, match="storage type"):
-        _check_grids(K.F64, grid(4), torch.zeros((4, 4), dtype=torch.float32).to_sparse())
+        _check_grids(K.F64, grid(4), torch.zeros((4, 4), dtype=torch.float32).to_sparse_csr())
     with pytest.raises(ValueError, match="unit column stride"):
         _check_grids(K.F64, torch.zeros(8, dtype=torch.float64))
