@@ -863,11 +863,12 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     // number of sweeps is.  Sweep 0 runs alone, untimed, unless it fits the
     // passes of the others and saves one: an even number of iterations takes
     // two passes, with sweep 0 one.  Measured with sweep 0 apart -> in the
-    // pass, both without the refresh of the other buffer below: star R=2 FP64 with init and norm, n = 30000, 100 iterations 42.1
-    // -> 37.9 ms, n = 1000, 10 iterations 81 -> 54 us; n = 16384, 2 / 50
-    // iterations, star R=1 FP32 2.91x / 1.45x, star R=8 BF16 1.19x / 1.01x,
-    // grid R=4 FP64 (the widest window) 1.14x / 1.01x.  A tiling override
-    // asks for the sweep kernel itself: one sweep per pass then.
+    // pass, both without the refresh of the other buffer below: star R=2 FP64
+    // with init and norm, n = 30000, 100 iterations 42.1 -> 37.9 ms, n = 1000,
+    // 10 iterations 81 -> 54 us; n = 16384, 2 / 50 iterations, star R=1 FP32
+    // 2.91x / 1.45x, star R=8 BF16 1.19x / 1.01x, grid R=4 FP64 (the widest
+    // window) 1.14x / 1.01x.  A tiling override asks for the sweep kernel
+    // itself: one sweep per pass then.
     const bool overridden = g_rows_per_wave > 0 || g_variant_override >= 0 || g_order >= 0 || g_wgs_per_cu >= 0;
     int alone = 1, passes = iterations;
     if (!overridden && pass_built(pattern, radius, dtype) && (p.mode != MODE_ELEM || dtype == BF16)) {
