@@ -251,7 +251,7 @@ static int launch_add(int dtype, int n, long long pitch, void *in, hipStream_t s
     // the stencil before it, go row by row too: with that stencil (FP64 star
     // R=1) n = 2000 28.6 us, flat 29.6; n = 700 10.0, flat 9.0.
     const long long bytes = count * (long long)dtype_size(dtype);
-    const bool l2_rows = vec && 2 * bytes > kInL2 && bytes <= 32ll << 20;
+    const bool l2_rows = vec && bytes > (6ll << 20) && bytes <= kL2s;
     if (pitch == n && (uintptr_t)in % 16 == 0 && launchable && !l2_rows) {
         return dtype == F64 ? launch_add_flat<F64>(count, in, s)
                : dtype == F32 ? launch_add_flat<F32>(count, in, s)

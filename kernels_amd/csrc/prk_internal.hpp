@@ -72,10 +72,7 @@ int launch_pass_f64(const SweepPlan &p, int sweeps, bool any, const void *in, vo
 int launch_pass_f32(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
 int launch_pass_bf16(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *out, hipStream_t s);
 
-constexpr long long kLastLevelCache = 256ll << 20;  // bytes
-// A call's arrays together up to this size stay in the L2s (32 MB in eight
-// dies) from one call to the next, however they were stored.
-constexpr long long kInL2 = 20ll << 20;
+constexpr long long kLastLevelCache = 256ll << 20, kL2s = 32ll << 20;  // bytes (the L2s of eight dies)
 
 // Sweeps of one pass at most: keeps a launch's time and the loss from an
 // interrupted one bounded (star R=2 FP64 at n = 30000: 256 sweeps take about

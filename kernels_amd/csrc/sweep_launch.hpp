@@ -107,25 +107,30 @@ int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipS
             }
         }
     }
-    // The other forms: arrays past the last-level cache, or in the L2s
-    // together, with the rows in flight and the non-temporal stores of the
-    // default fused sweep, arrays between (`cached`) with their stores through
-    // the cache.  Measured on MI355X, FP64 star R=2 unless said otherwise:
-    //  - unfused, then in += 1: n = 16384 1146 us temporal, 1071 non-temporal;
-    //    n = 1500 22.3, 25.6; n = 700 10.1, 9.4.
+    // The other forms take the rows in flight and the non-temporal stores of the
+    // default fused sweep where the call's arrays are past the caches or lie in
+    // the L2s together; between (`cached`) their stores go through the caches.
+    // Measured on MI355X, us, FP64 star R=2 unless said otherwise, in a loop on
+    // one grid / on three in turn:
+    //  - unfused, then in += 1: n = 1200 16.7 / 17.2, non-temporal 18.2 / 19.7;
+    //    n = 2300 40.2 / 40.4, 40.2 / 40.8; n = 3000 - / 75.6, - / 63.6; n = 700
+    //    10.1 / 10.6, 9.4 / 10.6; n = 16384 1146, 1071.
     //  - fused, ragged rows: FP64 inside the last-level cache takes element
-    //    stores (n = 2301 31.0 us, vectors 32.3, non-temporal ones 33.3; n =
-    //    4001 102, 91.8, 85.9), FP32 grid R=4 vectors (n = 4001 50.2,
-    //    non-temporal 60.7, element stores 49.1; star R=4, n = 1801 14.2, 15.3,
-    //    15.7), so does BF16 (stencils' mean at 4001 7 % over non-temporal).
-    //    The widest grids are bound by their arithmetic, and the vectors'
-    //    registers cost more than their stores save (FP64 grid R=8, n = 6501
-    //    809 us, vectors 849; FP32 grid R=8, n = 8001 402, 444).
+    //    stores (n = 2301 31.0, vectors 32.3, non-temporal ones 33.3; n = 4001
+    //    102, 91.8, 85.9; three grids in turn lose 4 to 14 % by it between 2301
+    //    and 3201, and are still as fast as before the vectors), FP32 grid R=4
+    //    vectors (n = 4001 50.2, non-temporal 60.7, element stores 49.1; star
+    //    R=4, n = 1801 14.2, 15.3, 15.7), so does BF16 (stencils' mean at 4001
+    //    7 % over non-temporal).  The widest grids are bound by their
+    //    arithmetic, and the vectors' registers cost more than their stores
+    //    save (FP64 grid R=8, n = 6501 809, vectors 849; FP32 grid R=8, n = 8001
+    //    402, 444).
     //  - fused, rows off 16 bytes: FP64 inside the last-level cache by element
-    //    (n = 3101 56.4 us, vectors 57.9, non-temporal 62.3).
+    //    (n = 3101 56.4, vectors 57.9, non-temporal 62.3).
     constexpr int PF = R > kRefMaxRadius ? 2 : 3;
     const long long bytes = (fuse ? 3 : 2) * (long long)p.span.nrows * p.pitch * (long long)sizeof(typename SweepGeom<DT, R>::T);
-    const bool fits = bytes <= kLastLevelCache, cached = fits && bytes > kInL2;
+    const bool fits = bytes <= kLastLevelCache;
+    const bool cached = fuse ? fits && bytes > (20ll << 20) : bytes > (12ll << 20) && bytes <= 2 * kL2s;
     if (fuse) {
         if (p.mode == MODE_RAGGED) {
             constexpr bool wide = P == GRID && R >= (DT == F64 ? 8 : DT == F32 ? 6 : kMaxRadius + 1);

@@ -64,7 +64,7 @@ def test_forms_by_size(gpu, oracle, dtype, n, pattern, radius):
 
 
 # the refresh alone and after a stencil takes rows or vectors of the array by its size
-@pytest.mark.parametrize("n", [1144, 1146, 2048, 2050])
+@pytest.mark.parametrize("n", [886, 888, 1144, 1146, 2048, 2050])
 def test_refresh_by_size(gpu, n):
     t = torch.rand((n, n), generator=torch.Generator(device=gpu).manual_seed(n), device=gpu, dtype=torch.float64)
     want = t + 1.0
