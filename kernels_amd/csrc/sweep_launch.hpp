@@ -113,8 +113,9 @@ int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipS
     // Measured on MI355X, us, FP64 star R=2 unless said otherwise, in a loop on
     // one grid / on three in turn:
     //  - unfused, then in += 1: n = 1200 16.7 / 17.2, non-temporal 18.2 / 19.7;
-    //    n = 2300 40.2 / 40.4, 40.2 / 40.8; n = 3000 - / 75.6, - / 63.6; n = 700
-    //    10.1 / 10.6, 9.4 / 10.6; n = 16384 1146, 1071.
+    //    n = 2300 40.2 / 40.4, 40.2 / 40.8; n = 3000 - / 75.6, - / 63.6 (three
+    //    pairs no longer fit the last-level cache); n = 700 10.1 / 10.6, 9.4 /
+    //    10.6; n = 16384 1146, 1071.
     //  - fused, ragged rows: FP64 inside the last-level cache takes element
     //    stores (n = 2301 31.0, vectors 32.3, non-temporal ones 33.3; n = 4001
     //    102, 91.8, 85.9; three grids in turn lose 4 to 14 % by it between 2301
@@ -130,7 +131,7 @@ int launch_pr(const SweepPlan &p, const void *in, void *in_next, void *out, hipS
     constexpr int PF = R > kRefMaxRadius ? 2 : 3;
     const long long bytes = (fuse ? 3 : 2) * (long long)p.span.nrows * p.pitch * (long long)sizeof(typename SweepGeom<DT, R>::T);
     const bool fits = bytes <= kLastLevelCache;
-    const bool cached = fuse ? fits && bytes > (20ll << 20) : bytes > (12ll << 20) && bytes <= 2 * kL2s;
+    const bool cached = fuse ? fits && bytes > (20ll << 20) : bytes > (12ll << 20) && bytes <= kLastLevelCache / 3;
     if (fuse) {
         if (p.mode == MODE_RAGGED) {
             constexpr bool wide = P == GRID && R >= (DT == F64 ? 8 : DT == F32 ? 6 : kMaxRadius + 1);
