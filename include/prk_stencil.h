@@ -160,12 +160,11 @@ int prk_l1norm_noalloc(int dtype, int n, long long pitch, int radius, const void
  * fused sweeps over the ping-pong pair (buf0 holds the initial in; buf1 is
  * scratch), timed with HIP events on `stream`.  Where the stencil's window
  * fits the registers the sweeps run many to a pass over the grid, with the
- * arithmetic of every sweep as it is one by one.  Sweep 0 runs before the
- * timed sweeps 1..iterations, unless it is part of the one pass that an even
- * number of iterations then takes.  *final_in_buf receives 0 or 1 (the buffer
- * holding in after the last refresh; iterations + 1 odd: 1), the other buffer
- * holds the in before it.  *avg_seconds: the mean time of one timed sweep, where
- * sweep 0 is in the pass that of all iterations + 1.  Synchronous. */
+ * arithmetic of every sweep as it is one by one.  One by one sweep 0 is
+ * untimed, in passes every sweep is timed.  *final_in_buf receives 0 or 1 (the
+ * buffer holding in after the last refresh; iterations + 1 odd: 1), the other
+ * buffer holds the in before it.  *avg_seconds: the mean time of one timed
+ * sweep.  Synchronous. */
 int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iterations,
             void *buf0, void *buf1, void *out, void *stream, int *final_in_buf,
             double *avg_seconds);

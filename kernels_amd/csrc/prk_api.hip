@@ -860,15 +860,14 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
     // The sweeps run in `passes` passes over the grid (pass.hpp) of nearly
     // equal length.  The final in must end in the buffer that one sweep per
     // pass would leave it in, so the number of passes is odd or even as the
-    // number of sweeps is.  Sweep 0 runs alone, untimed, unless it fits the
-    // passes of the others and saves one: an even number of iterations takes
-    // two passes, with sweep 0 one.  Measured with sweep 0 apart -> in the
-    // pass, both without the refresh of the other buffer below: star R=2 FP64
-    // with init and norm, n = 30000, 100 iterations 42.1 -> 37.9 ms, n = 1000,
-    // 10 iterations 81 -> 54 us; n = 16384, 2 / 50 iterations, star R=1 FP32
-    // 2.91x / 1.45x, star R=8 BF16 1.19x / 1.01x, grid R=4 FP64 (the widest
-    // window) 1.14x / 1.01x.  A tiling override asks for the sweep kernel
-    // itself: one sweep per pass then.
+    // number of sweeps is: an even number of iterations takes one pass, an odd
+    // one a pass and its last sweep alone.  The other buffer must hold the in
+    // before the final one, as after a sweep alone; after a pass the refreshes
+    // that the pass made on it are made in the buffer itself (one read and one
+    // write of the grid, where another sweep would take four).  Measured
+    // against two passes and a sweep: star R=2 FP64 with init and norm, n =
+    // 1000, 10 iterations 81 -> 56 us.  A tiling override asks for the sweep
+    // kernel itself: one sweep per pass then.
     const bool overridden = g_rows_per_wave > 0 || g_variant_override >= 0 || g_order >= 0 || g_wgs_per_cu >= 0;
     int alone = 1, passes = iterations;
     if (!overridden && pass_built(pattern, radius, dtype) && (p.mode != MODE_ELEM || dtype == BF16)) {
@@ -885,29 +884,37 @@ int prk_run(int pattern, int radius, int dtype, int n, long long pitch, int iter
             passes = apart;
         }
     }
-    const long long timed = (long long)iterations + 1 - alone;
+    const bool in_passes = passes + alone < (long long)iterations + 1;
+    const long long timed = (long long)iterations + 1 - (in_passes ? 0 : 1);
     void *bufs[2] = {buf0, buf1};
     int cur = 0;
-    if (alone) {
+    if (in_passes) {
+        // A process's first run would otherwise load its code between the events
+        // (0.6 ms, measured on a first run of n = 1000 whose passes take 20 us).
+        rc = launch_pass(p, 0, false, buf0, buf1, out, s);
+        p.load_only = true;
+        if (rc == PRK_OK && alone) rc = launch_sweep(p, buf0, buf1, out, s);
+        p.load_only = false;
+    } else {
         rc = launch_sweep(p, buf0, buf1, out, s);
         cur = 1;
     }
-    // A process's first pass would otherwise load its code between the events
-    // (0.6 ms, measured on a first run of n = 1000 whose passes take 20 us).
-    if (rc == PRK_OK && passes < timed) rc = launch_pass(p, 0, false, buf0, buf1, out, s);
     if (rc == PRK_OK) rc = check_hip(hipEventRecord(e0, s), "event record");
-    long long left = timed;
+    long long left = in_passes ? timed - alone : timed;
     int sweeps = 1;
     for (int it = 0; it < passes && rc == PRK_OK; ++it) {
         sweeps = (int)(left / (passes - it));  // spread over the passes left
         rc = sweeps == 1 ? launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s)
-                         : launch_pass(p, sweeps, !alone && it == 0, bufs[cur], bufs[cur ^ 1], out, s);
+                         : launch_pass(p, sweeps, it == 0, bufs[cur], bufs[cur ^ 1], out, s);
         left -= sweeps;
         cur ^= 1;
     }
-    // The buffer that the last pass read holds in as it was before all of the
-    // pass's refreshes; sweep by sweep it would hold the in before the last.
-    if (rc == PRK_OK && sweeps > 1) rc = launch_add_times(dtype, n, pitch, bufs[cur ^ 1], sweeps - 1, s);
+    if (rc == PRK_OK && in_passes && alone) {
+        rc = launch_sweep(p, bufs[cur], bufs[cur ^ 1], out, s);
+        cur ^= 1;
+    } else if (rc == PRK_OK && in_passes) {
+        rc = launch_add_times(dtype, n, pitch, bufs[cur ^ 1], sweeps - 1, s);
+    }
     if (rc == PRK_OK) rc = check_hip(hipEventRecord(e1, s), "event record");
     if (rc == PRK_OK) rc = check_hip(hipEventSynchronize(e1), "event sync");
     float ms = 0.0f;

@@ -26,6 +26,7 @@ struct SweepPlan {
     bool pad_writable;  // columns n..pitch-1 may be overwritten
     int order;          // workgroup -> tile order (sweep.hpp tile_of)
     int wgs_per_cu;     // occupancy cap, 0 = none
+    bool load_only = false;  // launch_sweep loads the kernel's code and launches nothing
 };
 
 // Number of fused-sweep variants: 0..5 the LDS-ring sweep (pipeline depth

@@ -11,6 +11,22 @@
 
 namespace prk {
 
+// Loads a kernel's code on the current device, so that a later launch does not
+// wait for it: asked for once per device (the answer takes 4 us).
+template <auto kernel>
+int load_code()
+{
+    static std::atomic<uint64_t> loaded{0};
+    int dev = 0;
+    int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
+    const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
+    if (rc || (loaded.load(std::memory_order_relaxed) & bit)) return rc;
+    hipFuncAttributes attr;
+    rc = check_hip(hipFuncGetAttributes(&attr, (const void *)kernel), "kernel load");
+    if (!rc) loaded.fetch_or(bit, std::memory_order_relaxed);
+    return rc;
+}
+
 template <int DT, int P, int R, bool FUSE, int MODE, int PF, int NT, bool RW = false>
 int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hipStream_t s)
 {
@@ -68,6 +84,10 @@ int launch_one(const SweepPlan &p, const void *in, void *in_next, void *out, hip
                 a.stash = 1;
             }
         }
+    }
+    if (p.load_only) {
+        if constexpr (RW) return load_code<sweep_rw_kernel<DT, P, R, FUSE, MODE, PF, NT>>();
+        else return load_code<sweep_kernel<DT, P, R, FUSE, MODE, PF, NT>>();
     }
     if constexpr (RW)
         hipLaunchKernelGGL((sweep_rw_kernel<DT, P, R, FUSE, MODE, PF, NT>), dim3(blocks), dim3(kThreads), dyn, s, a);
@@ -211,18 +231,8 @@ int launch_pass_pr(const SweepPlan &p, int sweeps, bool any, const void *in, voi
         const auto kernel =
             p.mode == MODE_VEC || p.mode == MODE_RAGGED ? pass_kernel<DT, P, R, true> : pass_kernel<DT, P, R, false>;
         if (sweeps == 0) {
-            // asked for once per device (the answer takes 4 us)
-            static std::atomic<uint64_t> loaded{0};
-            int dev = 0;
-            int rc = check_hip(hipGetDevice(&dev), "hipGetDevice");
-            const uint64_t bit = dev < 64 ? uint64_t(1) << dev : 0;
-            if (rc || (loaded.load(std::memory_order_relaxed) & bit)) return rc;
-            for (const auto k : {pass_kernel<DT, P, R, true>, pass_kernel<DT, P, R, false>}) {
-                hipFuncAttributes attr;
-                if (!rc) rc = check_hip(hipFuncGetAttributes(&attr, (const void *)k), "pass kernel load");
-            }
-            if (!rc) loaded.fetch_or(bit, std::memory_order_relaxed);
-            return rc;
+            const int rc = load_code<pass_kernel<DT, P, R, true>>();
+            return rc ? rc : load_code<pass_kernel<DT, P, R, false>>();
         }
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, a);
         return check_hip(hipGetLastError(), "pass launch");

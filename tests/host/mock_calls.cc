@@ -61,7 +61,7 @@ namespace prk {
 #define PRK_MOCK_DTYPE(d)                                                                                       \
     int launch_sweep_##d(const SweepPlan &p, const void *in, void *in_next, void *, hipStream_t)                \
     {                                                                                                           \
-        return record(p, 1, -1, in, in_next);                                                                   \
+        return p.load_only ? 0 : record(p, 1, -1, in, in_next);                                                 \
     }                                                                                                           \
     int launch_pass_##d(const SweepPlan &p, int sweeps, bool any, const void *in, void *in_next, void *, hipStream_t) \
     {                                                                                                           \

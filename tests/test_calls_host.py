@@ -190,3 +190,24 @@ def test_batch_heights_of_passes_are_not_tuned(lib):
         assert keys.value == 2 and L.mock_kernels() > 0
     finally:
         L.prk_batch_tuning_clear()
+
+
+@pytest.mark.parametrize("iterations", [1, 2, 3, 4, 10, 11, 255, 256, 257, 511, 512, 600])
+def test_run_of_passes_ends_in_its_buffer(lib, iterations):
+    # launches hand the in buffers over in turn, add up to iterations + 1
+    # sweeps, and end in the buffer that one sweep per launch would end in; a
+    # last sweep alone leaves the in before the last in the other buffer, after
+    # a pass that buffer is refreshed
+    L, n, final = lib, 512, C.c_int(-1)
+    p = [C.c_void_p(k << 30) for k in (1, 2, 3)]
+    L.mock_reset()
+    check(L, L.prk_run(0, 2, 0, n, C.c_longlong(n), iterations, *p, None, C.byref(final), None))
+    calls = sweeps(L)
+    assert sum(s[0] for s in calls) == iterations + 1 and final.value == (iterations + 1) % 2
+    src = 1 << 30
+    for s in calls:
+        assert s[5] == src and s[6] == (3 << 30) - src
+        src = s[6]
+    assert src == p[final.value].value
+    assert L.mock_kernels() == (0 if calls[-1][0] == 1 else 1)
+    assert all(s[1] == (s is calls[0]) for s in calls if s[0] > 1)  # the caller's values: the first pass alone
