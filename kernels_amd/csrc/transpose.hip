@@ -401,6 +401,11 @@ int launch_2h(TransposeArgs a, hipStream_t s)
 //  - Up to 4096 64 x 128 tiles, loads and stores through the caches: both
 //    matrices stay in the 256 MB of the last one (order 2000: 19; 4096: 79,
 //    93 non-temporal; 64 x 64 tiles in 8-byte accesses at 3001: 56, these 48).
+//    64 x 64 tiles between 1409 and 1600 and between 2497 and 2560, where the
+//    others come to little more than one or three workgroups for each CU
+//    (order 1495, 288 of them: 16.5, 64 x 64 14.0; 1450 14.7, 13.5; 2505
+//    38.4, 36.2; a little over two or four they stay ahead: 2101 27.9, 28.7;
+//    2901 49.6, 51.6).
 //  - Above, the same tiles, and only the stores non-temporal.  Rows on 64-byte
 //    boundaries share no cache line between tiles, so from 4800 on their loads
 //    are non-temporal too, with one workgroup at a time on a CU: order 32768
@@ -418,7 +423,8 @@ int launch_transpose(int order, double *A, double *B, hipStream_t s)
     const bool aligned = order % 2 == 0 && ptrs % 16 == 0;
     if (order > 4096 && !aligned) return launch_8b(a, s);
     const int nt = order <= 4096 ? NT_NONE : order >= 4800 && order % 8 == 0 && ptrs % 64 == 0 ? NT_ALL : NT_STORES;
-    const int shape = order <= 1024 ? 3 : 2;
+    const bool few = (order > 1408 && order <= 1600) || (order > 2496 && order <= 2560);
+    const int shape = order <= 1024 ? 3 : few ? 0 : 2;
     switch (g_tr_shape < 0 ? shape : g_tr_shape) {
     case 1: return launch_shape<128, 64>(a, nt, s);
     case 2: return launch_shape<64, 128>(a, nt, s);

@@ -13,7 +13,7 @@ import pytest
 
 ROOT = Path(__file__).resolve().parents[1]
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-SOURCES = [ROOT / "kernels_amd/csrc" / f for f in ("prk_api.hip", "batch.hip", "autotune.hip")]
+SOURCES = [ROOT / "kernels_amd/csrc" / f for f in ("prk_api.hip", "batch.hip", "autotune.hip", "transpose.hip")]
 SOURCES.append(ROOT / "tests/host/mock_calls.cc")
 
 pytestmark = pytest.mark.skipif(not (os.path.exists(HIPCC) and SOURCES[-1].exists()), reason="needs hipcc")
@@ -211,3 +211,15 @@ def test_run_of_passes_ends_in_its_buffer(lib, iterations):
     assert src == p[final.value].value
     assert L.mock_kernels() == (0 if calls[-1][0] == 1 else 1)
     assert all(s[1] == (s is calls[0]) for s in calls if s[0] > 1)  # the caller's values: the first pass alone
+
+
+@pytest.mark.parametrize("order,tiles", [
+    (1024, 32 * 16), (1408, 22 * 11), (1409, 23 * 23), (1495, 24 * 24), (1600, 25 * 25), (1601, 26 * 13),
+    (2496, 39 * 20), (2497, 40 * 40), (2560, 40 * 40), (2561, 41 * 21)])
+def test_transpose_tiles_where_turns_of_the_chip_end(lib, order, tiles):
+    # 64 x 128 tiles that come to little more than whole turns of the CUs left
+    # most of them idle (odd order 1495: 14.8 -> 16.5 us)
+    lib.mock_reset()
+    check(lib, lib.prk_transpose_ex(order, C.c_void_p(1 << 30), C.c_void_p(2 << 30), None))
+    (k,) = kernels(lib)
+    assert k[0] == tiles

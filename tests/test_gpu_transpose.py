@@ -128,3 +128,10 @@ def test_transpose_non_temporal_loads_edges(gpu, order, offset):
     # the line from which the loads of rows on 64-byte boundaries are
     # non-temporal, and matrices on 64 bytes (offset 0), 16 (2) and 8 (1)
     test_transpose_rule_edges(gpu, order, offset)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("order", [1408, 1409, 1410, 1471, 1600, 1601, 2496, 2497, 2560, 2561])
+def test_transpose_turns_edges(gpu, order, offset):
+    # the orders between which the tiles are 64 x 64
+    test_transpose_rule_edges(gpu, order, offset)
