@@ -282,7 +282,7 @@ def bench_batch(a) -> int:
         "dtype": "f32",
         "data": "synthetic (4096 seeded U(-1,1) grids, generator seed 7)",
         "config": {"workload": "batched uneven grids: 4096 solves, n log-uniform [64,2048], star/grid 50/50, "
-                               "R in 1..4, iterations 1..50, FP32 storage; one hipGraph of round launches",
+                               "R in 1..4, iterations 1..50, FP32 storage; one hipGraph",
                    "solves": len(specs), "launches_per_run": info["launches"], "tiles_per_run": info["tiles"],
                    "device_bytes": info["device_bytes"]},
         "effective_gbs": round(total_bytes * a.steps / (ms * 1e-3) / 1e9, 1),
@@ -812,7 +812,7 @@ def batch_section(a, torch, K) -> dict:
     solves_s = len(specs) / (ms * 1e-3)
     return {
         "workload": "4096 grids (seed 7): n log-uniform [64,2048], star/grid, R 1..4, iterations 1..50, "
-                    "FP32 storage, one hipGraph of round launches",
+                    "FP32 storage, one hipGraph",
         "solves_per_s": round(solves_s, 1), "ms_per_run": round(ms, 2), "runs": runs,
         "effective_gbs": round(sum(solve_bytes(s) for s in specs) / (ms * 1e-3) / 1e9, 1),
         "one_by_one_f64_solves_per_s": round(len(specs) / t64, 1),
