@@ -423,10 +423,11 @@ int prk_transpose_init(int order, double *A, double *B, void *stream);
 int prk_transpose_run(int order, int iterations, double *A, double *B, void *stream, double *avg_seconds);
 int prk_transpose_check(int order, int iterations, const double *B, double *abserr, void *stream);
 /* Tuning knob (process-wide, results unchanged): tile shape (rows x
- * columns of A, threads) 0 = 64x64, 1 = 128x64, 2 = 64x128 (default above
- * order 1024), 3 = 32x64 (default up to 1024), 4 = 128x128 on 1024 threads, 5 = 32x256, 6 = 256x32,
- * 7 = 64x128 on 512 threads, 8 = 128x128 on 1024 threads in two halves
- * of 64 KiB of LDS; tile order 0 = row-major (default), 1 =
+ * columns of A, threads) 0 = 64x64 (default from order 1409 to 1600 and from
+ * 2497 to 2560), 1 = 128x64, 2 = 64x128 (default at the other orders above
+ * 1024), 3 = 32x64 (default up to 1024), 4 = 128x128 on 1024 threads, 5 =
+ * 32x256, 6 = 256x32, 7 = 64x128 on 512 threads, 8 = 128x128 on 1024 threads
+ * in two halves of 64 KiB of LDS; tile order 0 = row-major (default), 1 =
  * column-major, 2 = groups of eight tile rows; -1 = default.  Above order
  * 4096 matrices whose rows are not on 16-byte boundaries always use 64x64
  * tiles with 8-byte accesses. */
