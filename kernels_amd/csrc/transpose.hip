@@ -88,8 +88,9 @@ __device__ inline void store2(__amdgpu_buffer_rsrc_t r, unsigned off, bool last,
     }
 }
 
-// Non-temporal accesses of a tile.
-enum { NT_NONE = 0, NT_STORES = 1, NT_ALL = 3 };
+// Non-temporal accesses of a tile.  NT_A: the stores of A alone, and B's rows
+// are loaded behind the barrier, after A's stores.
+enum { NT_NONE, NT_STORES, NT_A, NT_ALL };
 
 // One TR x TC tile of A (TR rows, TC columns) on NTH threads.
 template <int TR, int TC, int NTH, int NT, bool SPLIT>
@@ -98,7 +99,8 @@ __device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, do
     constexpr int LPR1 = TC / 2, RPP1 = NTH / LPR1, NP1 = TR / RPP1;  // A rows
     constexpr int LPR2 = TR / 2, RPP2 = NTH / LPR2, NP2 = TC / RPP2;  // B rows
     static_assert(NP1 >= 1 && NP2 >= 1 && RPP1 * NP1 == TR && RPP2 * NP2 == TC, "tile shape");
-    constexpr int AUX_LD = NT & 2 ? 2 : 0, AUX_ST = NT & 1 ? 2 : 0;
+    constexpr int AUX_LD = NT == NT_ALL ? 2 : 0;
+    constexpr int AUX_ST_A = NT == NT_NONE ? 0 : 2, AUX_ST_B = NT == NT_A ? 0 : AUX_ST_A;
     const int order = a.order;
     const unsigned row_bytes = (unsigned)order * 8u;
     union V { u32x4 v; double d[2]; };
@@ -129,16 +131,17 @@ __device__ inline void transpose_tile(const TransposeArgs &a, int tr, int tc, do
         z.d[1] = x[p].d[1] + 1.0;
         tile[p * RPP1 + ar][ac] = x[p].d[0];
         tile[p * RPP1 + ar][ac + 1] = x[p].d[1];
-        store2<AUX_ST, SPLIT>(ra, off_a + p * step_a, last_a, z.v);
+        store2<AUX_ST_A, SPLIT>(ra, off_a + p * step_a, last_a, z.v);
     }
+    if (NT == NT_A) __syncthreads();
 #pragma unroll
     for (int p = 0; p < NP2; ++p) y[p].v = load2<AUX_LD, SPLIT>(rb, off_b + p * step_b, last_b);
-    __syncthreads();
+    if (NT != NT_A) __syncthreads();
 #pragma unroll
     for (int p = 0; p < NP2; ++p) {
         y[p].d[0] = y[p].d[0] + tile[bc][p * RPP2 + br];
         y[p].d[1] = y[p].d[1] + tile[bc + 1][p * RPP2 + br];
-        store2<AUX_ST, SPLIT>(rb, off_b + p * step_b, last_b, y[p].v);
+        store2<AUX_ST_B, SPLIT>(rb, off_b + p * step_b, last_b, y[p].v);
     }
 }
 
@@ -371,6 +374,8 @@ int launch_shape(TransposeArgs a, int nt, hipStream_t s)
         hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_ALL, false>), dim3(blocks), dim3(NTH), dyn, s, a);
     else if (nt == NT_STORES)
         hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_STORES, false>), dim3(blocks), dim3(NTH), 0, s, a);
+    else if (nt == NT_A)
+        hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_A, false>), dim3(blocks), dim3(NTH), 0, s, a);
     else
         hipLaunchKernelGGL((transpose_kernel<TR, TC, NTH, NT_NONE, false>), dim3(blocks), dim3(NTH), 0, s, a);
     return check_hip(hipGetLastError(), "transpose launch");
@@ -410,10 +415,14 @@ int launch_2h(TransposeArgs a, hipStream_t s)
 //    boundaries share no cache line between tiles, so from 4800 on their loads
 //    are non-temporal too, with one workgroup at a time on a CU: order 32768
 //    6005 (two workgroups 6150, only the stores non-temporal 6540), 16384 1490
-//    (1520, 1630), 9000 529 (533, 598), 4808 150 (151 the stores alone; 4504
-//    112, 107).  Other rows lose by non-temporal loads (10002 817, 787).  32 x
-//    32 tiles without hints take them in between, but by where the rows fall on
-//    the memory's channels: 18 % faster at 21050, 18 % slower at 24006.
+//    (1520, 1630), 9000 529 (533, 598), 4808 150 (151 the stores alone).  Other
+//    rows lose by non-temporal loads (10002 817, 787).  32 x 32 tiles without hints
+//    take them in between, but by where the rows fall on the memory's channels:
+//    18 % faster at 21050, 18 % slower at 24006.
+//  - Up to 5200 the last-level cache holds much of what the tiles above leave:
+//    B's stores stay in it, and its loads wait for A's stores (4450 110, with
+//    B's non-temporal and its loads up front 121; 4590 121, 137; 4098 90.8,
+//    90.7; 5178 190, 191; above, the others are the faster: 7004 363, 352).
 //  - Odd orders and matrices off 16-byte boundaries: 64 x 64 tiles in 8-byte
 //    accesses (order 12289 1091, 64 x 128 1251).
 int launch_transpose(int order, double *A, double *B, hipStream_t s)
@@ -422,7 +431,8 @@ int launch_transpose(int order, double *A, double *B, hipStream_t s)
     const uintptr_t ptrs = (uintptr_t)A | (uintptr_t)B;
     const bool aligned = order % 2 == 0 && ptrs % 16 == 0;
     if (order > 4096 && !aligned) return launch_8b(a, s);
-    const int nt = order <= 4096 ? NT_NONE : order >= 4800 && order % 8 == 0 && ptrs % 64 == 0 ? NT_ALL : NT_STORES;
+    const bool lines = order % 8 == 0 && ptrs % 64 == 0;
+    const int nt = order <= 4096 ? NT_NONE : lines && order >= 4800 ? NT_ALL : order <= 5200 ? NT_A : NT_STORES;
     const bool few = (order > 1408 && order <= 1600) || (order > 2496 && order <= 2560);
     const int shape = order <= 1024 ? 3 : few ? 0 : 2;
     switch (g_tr_shape < 0 ? shape : g_tr_shape) {

@@ -135,3 +135,11 @@ def test_transpose_non_temporal_loads_edges(gpu, order, offset):
 def test_transpose_turns_edges(gpu, order, offset):
     # the orders between which the tiles are 64 x 64
     test_transpose_rule_edges(gpu, order, offset)
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("order", [4450, 4606, 5198, 5200, 5202])
+def test_transpose_cached_b_edges(gpu, order, offset):
+    # even orders up to 5200 keep B's stores in the last-level cache and load
+    # its rows behind the barrier
+    test_transpose_rule_edges(gpu, order, offset)
